@@ -16,6 +16,7 @@
 #include <cmath>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/hyqmom.h"
@@ -84,17 +85,16 @@ __device__ __forceinline__ float dgelu(float z) {
   return s + z * s * (1.0f - s) * 1.5957691216057308f * (1.0f + 0.134145f * z * z);
 }
 
-// C[M x N] = A[M x K] . B[K x N] (+ bias), A(m,k) = A[m*sam + k*sak], B(k,n) = B[k*sbk + n*sbn].
+// H[M x N] = act(A[M x K] . B[K x N] + bias), row-major A (leading dimension lda), B (ldb), H (ldc).
 // One wave computes rows [16 r, 16 r + 16) x columns [16 NT c, 16 NT (c+1)); lane l feeds
 // A rows l%16 and B columns l%16 with the eight k values 8(l/16)..+7 of each 32-wide k step,
 // and receives D rows 4(l/16)..+3 of column l%16.
-// Epilogue: act 0 = none, 1 = GELU; Z gets the pre-activation, H the activation (either may
-// be null); stores only rows < M and columns < Nst.
+// Epilogue: act 0 = none, 1 = GELU; stores only rows < M.
 template <int NT>
-__global__ __launch_bounds__(256) void k_gemm(const float* __restrict__ A, long sam, long sak,
-                                              const float* __restrict__ B, long sbk, long sbn,
-                                              int M, int N, int K, const float* __restrict__ bias,
-                                              float* Z, float* H, long ldc, int Nst, int act) {
+__global__ __launch_bounds__(256) void k_gemm(const float* __restrict__ A, long lda,
+                                              const float* __restrict__ B, long ldb, int M, int N,
+                                              int K, const float* __restrict__ bias,
+                                              float* __restrict__ H, long ldc, int act) {
   const int lane = threadIdx.x & 63;
   const long rt = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int ct = blockIdx.y;
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(256) void k_gemm(const float* __restrict__ A, long 
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int k = k0 + 8 * q + e;
-      const float v = (row < M && k < K) ? A[row * sam + (long)k * sak] : 0.f;
+      const float v = (row < M && k < K) ? A[row * lda + k] : 0.f;
       a[e] = f2bf(v);
     }
 #pragma unroll
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(256) void k_gemm(const float* __restrict__ A, long 
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const int k = k0 + 8 * q + e;
-        const float v = (col < N && k < K) ? B[(long)k * sbk + col * sbn] : 0.f;
+        const float v = (col < N && k < K) ? B[k * ldb + col] : 0.f;
         b[e] = f2bf(v);
       }
       acc[t] = mfma32(a, b, acc[t]);
@@ -128,25 +128,18 @@ __global__ __launch_bounds__(256) void k_gemm(const float* __restrict__ A, long 
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const long col = (long)(ct * NT + t) * 16 + r;
-    if (col >= Nst) continue;
-    const float bv = bias ? bias[col] : 0.f;
+    if (col >= N) continue;
+    const float bv = bias[col];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const long orow = rt * 16 + 4 * q + e;
       if (orow >= M) continue;
       const float z = acc[t][e] + bv;
-      if (Z) Z[orow * ldc + col] = z;
-      if (H) H[orow * ldc + col] = act == 1 ? gelu(z) : z;
+      H[orow * ldc + col] = act == 1 ? gelu(z) : z;
     }
   }
 }
 
-// dZ = dH * GELU'(Z)
-__global__ void k_gelu_bwd(const float* __restrict__ Z, float* __restrict__ dH, long n) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  dH[i] *= dgelu(Z[i]);
-}
 // normalized features: Xn[b][j] = (X[b][j] - mu[j]) / sd[j]  (j < 15), 0 for j = 15
 __global__ void k_normalize(const float* __restrict__ X, const float* __restrict__ stat,
                             float* __restrict__ Xn, long n) {
@@ -154,39 +147,6 @@ __global__ void k_normalize(const float* __restrict__ X, const float* __restrict
   if (i >= n * 16) return;
   const int j = (int)(i & 15);
   Xn[i] = j < 15 ? (X[i] - stat[j]) / stat[16 + j] : 0.0f;
-}
-// loss gradient of L = 1/(2B) sum (Y - Tn)^2 on the two outputs; Y rows of 16.
-__global__ void k_mse_grad(const float* __restrict__ Y, const float* __restrict__ T,
-                           const float* __restrict__ ystat, float* __restrict__ dY, long n,
-                           float* loss) {
-  const long b = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  float l = 0.f;
-  if (b < n) {
-    for (int o = 0; o < 16; ++o) dY[b * 16 + o] = 0.f;
-    for (int o = 0; o < 2; ++o) {
-      const float tn = (T[b * 2 + o] - ystat[o]) / ystat[2 + o];
-      const float d = Y[b * 16 + o] - tn;
-      dY[b * 16 + o] = d / (float)n;
-      l += 0.5f * d * d / (float)n;
-    }
-  }
-  // wave reduction then one atomic per wave
-  for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
-  if ((threadIdx.x & 63) == 0) atomicAdd(loss, l);
-}
-__global__ void k_colsum(const float* __restrict__ D, long n, int ncol, float* __restrict__ out) {
-  const int c = blockIdx.x;
-  float s = 0.f;
-  for (long b = threadIdx.x; b < n; b += blockDim.x) s += D[b * ncol + c];
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  __shared__ float red[16];
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float t = 0.f;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += red[w];
-    out[c] = t;
-  }
 }
 __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
                        float* __restrict__ v, long n, float lr, float b1, float b2, float eps,
@@ -492,6 +452,253 @@ __global__ __launch_bounds__(64 * WAVES) void k_mlp_fused(const void* __restrict
   }
 }
 
+// ---- training: forward, loss and gradients in three launches ---------------------------------
+// The layer-by-layer form this replaces took 20 launches, and its weight gradients, products
+// over the batch with 32 x 32 results, ran on one block each: 0.4 to 1 ms a product at 8192
+// rows.  Here k_train_rows takes 16 rows per wave through all layers and back, k_wgrad splits
+// the batch of every weight gradient over waves, and k_grad_sum adds the parts in a fixed
+// order.  A call at 8192 rows and width 32: 4171 -> 71 us, of which the three kernels take 10,
+// 5 and 6 us (latency of the six chained products; the operands' 3.7 MB stay in L2) and the
+// host's synchronization and read-back the rest.  Operands are rounded to bf16 and sums kept
+// in FP32 as before.
+//
+// Transposed weights in MFMA B-operand order for the backward products (dA = dZ W^T): for
+// k-step ks and column tile t, lane l holds W[16 t + l % 16][32 ks + 8 (l / 16) + e], zero
+// past the layer's columns.
+constexpr int PT_W4 = 0;                        // 1 k-step (16 outputs, padded) x NTH tiles
+constexpr int PT_W3 = PT_W4 + NTH * 512;        // KSH x NTH
+constexpr int PT_W2 = PT_W3 + KSH * NTH * 512;
+constexpr int PT_N = PT_W2 + KSH * NTH * 512;
+__global__ void k_pack_t(const float* __restrict__ p, short* __restrict__ pk) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= PT_N) return;
+  int base, cols;
+  const float* W;
+  if (i < PT_W3) { base = PT_W4; cols = OUT; W = p + OFF_W4; }
+  else if (i < PT_W2) { base = PT_W3; cols = HID; W = p + OFF_W3; }
+  else { base = PT_W2; cols = HID; W = p + OFF_W2; }
+  const int o = i - base, chunk = o / 512, r = o % 512, lane = r / 8, e = r % 8;
+  const int ks = chunk / NTH, t = chunk % NTH;
+  const int row = 16 * t + lane % 16, col = 32 * ks + 8 * (lane / 16) + e;
+  pk[i] = col < cols ? f2bf(W[row * cols + col]) : (short)0;
+}
+
+// Batch operands of the weight gradients, bf16, one row per feature: [feature][npad samples],
+// so that an MFMA lane reads its eight samples as one 16-byte load.
+constexpr int TR_X = 0, TR_H = TR_X + IN, TR_DZ = TR_H + 3 * HID, TR_DY = TR_DZ + 3 * HID,
+              TR_N = TR_DY + OUT;  // rows of the operand buffer
+constexpr int NBIAS = 3 * HID + OUT + 1;  // bias gradients b1 b2 b3 b4 and the loss, per block
+constexpr int kRowWaves = 4;
+
+// One wave per 16 rows: forward (as the fused inference), loss gradient, and back to dZ1,
+// with the pre-activations in registers; writes the operands of the weight gradients and the
+// block's part of the bias gradients and the loss.  Rows past n (up to npad) give zeros.
+__global__ __launch_bounds__(64 * kRowWaves) void k_train_rows(
+    const float* __restrict__ X, const float* __restrict__ T, long n, long npad,
+    const float* __restrict__ p, const short* __restrict__ pk, const short* __restrict__ pt,
+    short* __restrict__ tr, float* __restrict__ part) {
+  __shared__ __align__(16) short act[kRowWaves][16 * ACT_LD];
+  __shared__ float red[kRowWaves][NBIAS];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
+  const s8* W = reinterpret_cast<const s8*>(pk);
+  const s8* Wt = reinterpret_cast<const s8*>(pt);
+  short* A = act[w];
+  float bsum[3][NTH], ysum = 0.f, loss = 0.f;
+#pragma unroll
+  for (int L = 0; L < 3; ++L)
+#pragma unroll
+    for (int t = 0; t < NTH; ++t) bsum[L][t] = 0.f;
+  typedef short s4 __attribute__((ext_vector_type(4)));
+  // four rows 4q..4q+3 of one column as bf16: to the operand buffer and to the wave's tile
+  auto put = [&](int row_of_tr, long row0, int t, const float* v, bool tile) {
+    s4 h;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) h[e] = f2bf(v[e]);
+    *reinterpret_cast<s4*>(&tr[(size_t)(row_of_tr + 16 * t + r) * npad + row0 + 4 * q]) = h;
+    if (tile)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) A[(4 * q + e) * ACT_LD + 16 * t + r] = h[e];
+  };
+  for (long tile = (long)blockIdx.x * kRowWaves + w; tile * 16 < npad; tile += (long)gridDim.x * kRowWaves) {
+    const long row0 = tile * 16, row = row0 + r;
+    int wl = lane;  // not an invariant of the loop: the weights' loads stay in it
+    asm volatile("" : "+v"(wl));
+    f4 z[3][NTH];
+    {
+      s8 a;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int k = 8 * q + e;
+        float v = 0.f;
+        if (row < n && k < 15) v = (X[row * 16 + k] - p[OFF_XMU + k]) / p[OFF_XSD + k];
+        a[e] = f2bf(v);
+        if (q < 2) tr[(size_t)(TR_X + k) * npad + row] = a[e];
+      }
+#pragma unroll
+      for (int t = 0; t < NTH; ++t) z[0][t] = mfma32(a, W[PK_W1 / 8 + t * 64 + wl], f4{0.f, 0.f, 0.f, 0.f});
+    }
+    // (a generic lambda per layer: every index of z is then a constant whatever the width)
+    auto forward = [&](auto layer) {
+      constexpr int L = decltype(layer)::value;
+      const int ob = L == 0 ? (int)OFF_B1 : (L == 1 ? (int)OFF_B2 : (int)OFF_B3);
+      if (L > 0) {
+        const int wb = (L == 1 ? PK_W2 : PK_W3) / 8;
+#pragma unroll
+        for (int t = 0; t < NTH; ++t) z[L][t] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KSH; ++ks) {
+          const s8 av = *reinterpret_cast<const s8*>(&A[r * ACT_LD + 32 * ks + 8 * q]);
+#pragma unroll
+          for (int t = 0; t < NTH; ++t) z[L][t] = mfma32(av, W[wb + (ks * NTH + t) * 64 + wl], z[L][t]);
+        }
+        wave_lds_fence();  // every lane has read the tile before it is overwritten
+      }
+#pragma unroll
+      for (int t = 0; t < NTH; ++t) {
+        const float b = p[ob + 16 * t + r];
+        float h[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          z[L][t][e] += b;
+          h[e] = gelu(z[L][t][e]);
+        }
+        put(TR_H + L * HID, row0, t, h, true);
+      }
+      wave_lds_fence();
+    };
+    forward(std::integral_constant<int, 0>{});
+    forward(std::integral_constant<int, 1>{});
+    forward(std::integral_constant<int, 2>{});
+    // outputs and the loss gradient (columns 0 and 1; the others are zero)
+    f4 y = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KSH; ++ks)
+      y = mfma32(*reinterpret_cast<const s8*>(&A[r * ACT_LD + 32 * ks + 8 * q]),
+                 W[PK_W4 / 8 + ks * 64 + wl], y);
+    float dy[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const long ro = row0 + 4 * q + e;
+      dy[e] = 0.f;
+      if (r < 2 && ro < n) {
+        const float tn = (T[ro * 2 + r] - p[OFF_YMU + r]) / p[OFF_YSD + r];
+        const float d = (y[e] + p[OFF_B4 + r]) - tn;
+        dy[e] = d / (float)n;
+        loss += 0.5f * d * d / (float)n;
+        ysum += dy[e];
+      }
+    }
+    wave_lds_fence();  // the tile's activations are read: dY takes its place
+    put(TR_DY, row0, 0, dy, true);
+    wave_lds_fence();
+    // back: dA = dZ W^T, dZ = dA GELU'(Z)
+    auto backward = [&](auto layer) {
+      constexpr int L = decltype(layer)::value;
+      f4 d[NTH];
+#pragma unroll
+      for (int t = 0; t < NTH; ++t) d[t] = f4{0.f, 0.f, 0.f, 0.f};
+      if (L == 2) {
+        // 16 columns of dY: k-step columns 16..31 are not there
+        const s8 av = q < 2 ? *reinterpret_cast<const s8*>(&A[r * ACT_LD + 8 * q]) : s8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int t = 0; t < NTH; ++t) d[t] = mfma32(av, Wt[PT_W4 / 8 + t * 64 + wl], d[t]);
+      } else {
+        const int wb = (L == 1 ? PT_W3 : PT_W2) / 8;
+#pragma unroll
+        for (int ks = 0; ks < KSH; ++ks) {
+          const s8 av = *reinterpret_cast<const s8*>(&A[r * ACT_LD + 32 * ks + 8 * q]);
+#pragma unroll
+          for (int t = 0; t < NTH; ++t) d[t] = mfma32(av, Wt[wb + (ks * NTH + t) * 64 + wl], d[t]);
+        }
+      }
+      wave_lds_fence();
+#pragma unroll
+      for (int t = 0; t < NTH; ++t) {
+        float g[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          g[e] = d[t][e] * dgelu(z[L][t][e]);
+          bsum[L][t] += g[e];
+        }
+        put(TR_DZ + L * HID, row0, t, g, L > 0);
+      }
+      wave_lds_fence();
+    };
+    backward(std::integral_constant<int, 2>{});
+    backward(std::integral_constant<int, 1>{});
+    backward(std::integral_constant<int, 0>{});
+  }
+  // the block's bias gradients and loss: over a wave's four row quarters, then over the waves
+#pragma unroll
+  for (int L = 0; L < 3; ++L)
+#pragma unroll
+    for (int t = 0; t < NTH; ++t) {
+      float v = bsum[L][t];
+      v += __shfl_xor(v, 16);
+      v += __shfl_xor(v, 32);
+      if (q == 0) red[w][L * HID + 16 * t + r] = v;
+    }
+  ysum += __shfl_xor(ysum, 16);
+  ysum += __shfl_xor(ysum, 32);
+  if (q == 0) red[w][3 * HID + r] = ysum;
+  for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o);
+  if (lane == 0) red[w][NBIAS - 1] = loss;
+  __syncthreads();
+  for (int i = threadIdx.x; i < NBIAS; i += 64 * kRowWaves) {
+    float v = 0.f;
+    for (int u = 0; u < kRowWaves; ++u) v += red[u][i];
+    part[(size_t)blockIdx.x * NBIAS + i] = v;
+  }
+}
+
+// Weight gradients G = H^T dZ of all four layers, split over the batch: wave (tile, chunk)
+// adds one 16 x 16 tile of one layer's gradient over `rows` samples (a multiple of 32) and
+// writes it to the chunk's part [NPARAM].
+constexpr int WT1 = NTH, WT2 = WT1 + NTH * NTH, WT3 = WT2 + NTH * NTH, WT_N = WT3 + NTH;  // tiles
+__global__ __launch_bounds__(256) void k_wgrad(const short* __restrict__ tr, long npad, int rows,
+                                               float* __restrict__ part) {
+  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const int tile = blockIdx.y * 4 + (threadIdx.x >> 6);
+  if (tile >= WT_N) return;
+  int a, b, ra, rb, ldc;  // tile (a, b): operand rows ra + 16 a, rb + 16 b; the gradient's columns
+  size_t off;
+  if (tile < WT1) { a = 0; b = tile; ra = TR_X; rb = TR_DZ; off = OFF_W1; ldc = HID; }
+  else if (tile < WT2) { a = (tile - WT1) / NTH; b = (tile - WT1) % NTH; ra = TR_H; rb = TR_DZ + HID; off = OFF_W2; ldc = HID; }
+  else if (tile < WT3) { a = (tile - WT2) / NTH; b = (tile - WT2) % NTH; ra = TR_H + HID; rb = TR_DZ + 2 * HID; off = OFF_W3; ldc = HID; }
+  else { a = tile - WT3; b = 0; ra = TR_H + 2 * HID; rb = TR_DY; off = OFF_W4; ldc = OUT; }
+  const long k0 = (long)blockIdx.x * rows, k1 = k0 + rows < npad ? k0 + rows : npad;
+  const s8* pa = reinterpret_cast<const s8*>(tr + (size_t)(ra + 16 * a + r) * npad);
+  const s8* pb = reinterpret_cast<const s8*>(tr + (size_t)(rb + 16 * b + r) * npad);
+  f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (long k = k0; k < k1; k += 32) acc = mfma32(pa[k / 8 + q], pb[k / 8 + q], acc);
+  float* o = part + (size_t)blockIdx.x * NPARAM + off;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[(16 * a + 4 * q + e) * ldc + 16 * b + r] = acc[e];
+}
+
+// The gradient: every parameter's parts added in order (weights: k_wgrad's chunks; biases
+// and the loss: k_train_rows' blocks).
+__global__ void k_grad_sum(const float* __restrict__ wpart, int nw, const float* __restrict__ bpart,
+                           int nb, float* __restrict__ g, float* __restrict__ loss) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i > (int)NPARAM) return;
+  int bias = -1;
+  if (i == (int)NPARAM) bias = NBIAS - 1;
+  else if (i >= (int)OFF_B1 && i < (int)OFF_W2) bias = i - (int)OFF_B1;
+  else if (i >= (int)OFF_B2 && i < (int)OFF_W3) bias = HID + i - (int)OFF_B2;
+  else if (i >= (int)OFF_B3 && i < (int)OFF_W4) bias = 2 * HID + i - (int)OFF_B3;
+  else if (i >= (int)OFF_B4) bias = 3 * HID + i - (int)OFF_B4;
+  const float* src = bias >= 0 ? bpart + bias : wpart + i;
+  const size_t st = bias >= 0 ? NBIAS : NPARAM;
+  const int m = bias >= 0 ? nb : nw;
+  float v = 0.f;
+#pragma unroll 8
+  for (int k = 0; k < m; ++k) v += src[(size_t)k * st];
+  if (i == (int)NPARAM) *loss = v;
+  else g[i] = v;
+}
+
 // Launch shapes of the fused inference (waves per block, row tiles per wave): 16 x 1, 8 x 2
 // (each B operand feeding two MFMAs) and 8 x 1 (smaller blocks, so that more of them share a
 // CU).  They compute the same values in the same order; the first large inference times them
@@ -531,11 +738,11 @@ void launch_fused(int shape, bool mask, bool bin, const void* X, long n, const f
 unsigned g1(long n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
 template <int NT>
-void gemm(hipStream_t s, const float* A, long sam, long sak, const float* B, long sbk, long sbn,
-          long M, int N, long K, const float* bias, float* Z, float* H, long ldc, int Nst, int act) {
+void gemm(hipStream_t s, const float* A, long lda, const float* B, long ldb, long M, int N, int K,
+          const float* bias, float* H, long ldc, int act) {
   dim3 grid((unsigned)((M + 63) / 64), (unsigned)((N + 16 * NT - 1) / (16 * NT)));
-  hipLaunchKernelGGL((k_gemm<NT>), grid, dim3(256), 0, s, A, sam, sak, B, sbk, sbn, (int)M, N,
-                     (int)K, bias, Z, H, ldc, Nst, act);
+  hipLaunchKernelGGL((k_gemm<NT>), grid, dim3(256), 0, s, A, lda, B, ldb, (int)M, N, K, bias,
+                     H, ldc, act);
 }
 
 struct Net {
@@ -543,8 +750,11 @@ struct Net {
   float* grad;   // NPARAM
   float* m1;     // Adam moments
   float* m2;
-  long cap;      // training activation capacity (samples)
-  float *Xn, *Z1, *H1, *Z2, *H2, *Z3, *H3, *Y, *dY, *dA, *dB;
+  long cap;      // training capacity (samples, padded)
+  short* tr;     // [TR_N][cap] operands of the weight gradients
+  float *wpart, *bpart;  // gradient parts: [chunks][NPARAM], [blocks][NBIAS]
+  short* tpack;  // training's packed bf16 weights, on m->stream: as packed, then transposed
+  long tpack_version;
   long icap;     // inference capacity: normalized input, two hidden ping-pong buffers, output
   float *iX, *iA, *iB, *iY;
   float* loss;
@@ -570,52 +780,31 @@ static int ensure_icap(Net* m, long n) {
   return HYQ_OK;
 }
 
-static int ensure_cap(Net* m, long n) {
-  if (n <= m->cap) return HYQ_OK;
-  float** bufs[] = {&m->Xn, &m->Z1, &m->H1, &m->Z2, &m->H2, &m->Z3, &m->H3, &m->Y, &m->dY, &m->dA, &m->dB};
-  const long width[] = {IN, HID, HID, HID, HID, HID, HID, OUT, OUT, HID, HID};
-  for (int i = 0; i < 11; ++i) {
-    (void)hipFree(*bufs[i]);
-    *bufs[i] = nullptr;
-    if (hipMalloc(bufs[i], sizeof(float) * width[i] * n) != hipSuccess)
-      return mfail(HYQ_ENOMEM, "mlp activation allocation");
-  }
-  m->cap = n;
+// Rows of the batch per part of the weight gradients, and blocks of k_train_rows: enough of
+// both to fill the chip at a training batch (8192 rows: 32 parts, 128 blocks), few enough
+// that adding them stays short.
+static long train_pad(long n) { return (n + 31) / 32 * 32; }
+static int wgrad_rows(long npad) {
+  const long r = (npad + 63) / 64;  // at most 64 parts
+  return (int)((std::max<long>(r, 256) + 31) / 32 * 32);
+}
+static int wgrad_parts(long npad) { return (int)((npad + wgrad_rows(npad) - 1) / wgrad_rows(npad)); }
+static int row_blocks(long npad) { return (int)std::min<long>((npad / 16 + kRowWaves - 1) / kRowWaves, 256); }
+
+static int ensure_cap(Net* m, long npad) {
+  if (npad <= m->cap) return HYQ_OK;
+  (void)hipFree(m->tr);
+  (void)hipFree(m->wpart);
+  (void)hipFree(m->bpart);
+  m->tr = nullptr;
+  m->wpart = m->bpart = nullptr;
+  m->cap = 0;
+  if (hipMalloc(&m->tr, sizeof(short) * TR_N * npad) != hipSuccess ||
+      hipMalloc(&m->wpart, sizeof(float) * NPARAM * 64) != hipSuccess ||
+      hipMalloc(&m->bpart, sizeof(float) * NBIAS * 256) != hipSuccess)
+    return mfail(HYQ_ENOMEM, "mlp training allocation");
+  m->cap = npad;
   return HYQ_OK;
-}
-
-// forward on normalized inputs m->Xn (n rows); fills Z*, H*, Y
-static void forward(Net* m, long n) {
-  const float* p = m->blob;
-  gemm<NTH>(m->stream, m->Xn, IN, 1, p + OFF_W1, HID, 1, n, HID, IN, p + OFF_B1, m->Z1, m->H1, HID, HID, 1);
-  gemm<NTH>(m->stream, m->H1, HID, 1, p + OFF_W2, HID, 1, n, HID, HID, p + OFF_B2, m->Z2, m->H2, HID, HID, 1);
-  gemm<NTH>(m->stream, m->H2, HID, 1, p + OFF_W3, HID, 1, n, HID, HID, p + OFF_B3, m->Z3, m->H3, HID, HID, 1);
-  gemm<1>(m->stream, m->H3, HID, 1, p + OFF_W4, OUT, 1, n, OUT, HID, p + OFF_B4, nullptr, m->Y, OUT, OUT, 0);
-}
-
-// gradients of the loss into m->grad (forward must have run)
-static void backward(Net* m, long n) {
-  const float* p = m->blob;
-  float* g = m->grad;
-  hipStream_t s = m->stream;
-  // layer 4
-  gemm<1>(s, m->H3, 1, HID, m->dY, OUT, 1, HID, OUT, n, nullptr, nullptr, g + OFF_W4, OUT, OUT, 0);
-  hipLaunchKernelGGL(k_colsum, dim3(OUT), dim3(256), 0, s, m->dY, n, OUT, g + OFF_B4);
-  gemm<NTH>(s, m->dY, OUT, 1, p + OFF_W4, 1, OUT, n, HID, OUT, nullptr, nullptr, m->dA, HID, HID, 0);
-  hipLaunchKernelGGL(k_gelu_bwd, dim3(g1(n * HID)), dim3(256), 0, s, m->Z3, m->dA, n * HID);
-  // layer 3
-  gemm<NTH>(s, m->H2, 1, HID, m->dA, HID, 1, HID, HID, n, nullptr, nullptr, g + OFF_W3, HID, HID, 0);
-  hipLaunchKernelGGL(k_colsum, dim3(HID), dim3(256), 0, s, m->dA, n, HID, g + OFF_B3);
-  gemm<NTH>(s, m->dA, HID, 1, p + OFF_W3, 1, HID, n, HID, HID, nullptr, nullptr, m->dB, HID, HID, 0);
-  hipLaunchKernelGGL(k_gelu_bwd, dim3(g1(n * HID)), dim3(256), 0, s, m->Z2, m->dB, n * HID);
-  // layer 2
-  gemm<NTH>(s, m->H1, 1, HID, m->dB, HID, 1, HID, HID, n, nullptr, nullptr, g + OFF_W2, HID, HID, 0);
-  hipLaunchKernelGGL(k_colsum, dim3(HID), dim3(256), 0, s, m->dB, n, HID, g + OFF_B2);
-  gemm<NTH>(s, m->dB, HID, 1, p + OFF_W2, 1, HID, n, HID, HID, nullptr, nullptr, m->dA, HID, HID, 0);
-  hipLaunchKernelGGL(k_gelu_bwd, dim3(g1(n * HID)), dim3(256), 0, s, m->Z1, m->dA, n * HID);
-  // layer 1
-  gemm<NTH>(s, m->Xn, 1, IN, m->dA, HID, 1, IN, HID, n, nullptr, nullptr, g + OFF_W1, HID, HID, 0);
-  hipLaunchKernelGGL(k_colsum, dim3(HID), dim3(256), 0, s, m->dA, n, HID, g + OFF_B1);
 }
 
 }  // namespace
@@ -653,11 +842,12 @@ int create(const float* blob_host, void** out) {
   MCHK(hipMemset(m->m1, 0, sizeof(float) * NPARAM), "adam m");
   MCHK(hipMemset(m->m2, 0, sizeof(float) * NPARAM), "adam v");
   MCHK(hipMalloc(&m->packed, sizeof(short) * PK_N), "mlp packed weights");
+  MCHK(hipMalloc(&m->tpack, sizeof(short) * (PK_N + PT_N)), "mlp packed weights");
   m->shape = -1;
   MCHK(hipEventCreate(&m->ev[0]), "mlp event");
   MCHK(hipEventCreate(&m->ev[1]), "mlp event");
   m->version = 1;
-  m->packed_version = 0;
+  m->packed_version = m->tpack_version = 0;
   *out = m;
   return HYQ_OK;
 }
@@ -666,10 +856,11 @@ int destroy(void* h) {
   Net* m = static_cast<Net*>(h);
   if (!m) return HYQ_OK;
   (void)hipStreamSynchronize(m->stream);
-  float* bufs[] = {m->blob, m->grad, m->m1, m->m2, m->loss, m->Xn, m->Z1, m->H1, m->Z2,
-                   m->H2, m->Z3, m->H3, m->Y, m->dY, m->dA, m->dB, m->iX, m->iA, m->iB, m->iY};
+  float* bufs[] = {m->blob, m->grad, m->m1, m->m2, m->loss, m->wpart, m->bpart, m->iX, m->iA, m->iB, m->iY};
   for (float* b : bufs) (void)hipFree(b);
   (void)hipFree(m->packed);
+  (void)hipFree(m->tpack);
+  (void)hipFree(m->tr);
   for (hipEvent_t e : m->ev)
     if (e) (void)hipEventDestroy(e);
   (void)hipStreamDestroy(m->stream);
@@ -789,8 +980,8 @@ int set_shape(void* h, int32_t shape) {
   return HYQ_OK;
 }
 
-// The same prediction through the layer-by-layer GEMM kernels of training (a cross-check
-// of the fused kernel).
+// The same prediction through the layer-by-layer GEMM kernels (a cross-check of the fused
+// kernel).
 int infer_layers(void* h, const float* X, int64_t n, float* P) {
   Net* m = static_cast<Net*>(h);
   if (!m || !X || !P || n < 0) return mfail(HYQ_EINVAL, "bad argument");
@@ -800,10 +991,10 @@ int infer_layers(void* h, const float* X, int64_t n, float* P) {
   const float* p = m->blob;
   hipStream_t stream = m->stream;
   hipLaunchKernelGGL(k_normalize, dim3(g1(n * 16)), dim3(256), 0, stream, X, p + OFF_XMU, m->iX, (long)n);
-  gemm<NTH>(stream, m->iX, IN, 1, p + OFF_W1, HID, 1, n, HID, IN, p + OFF_B1, nullptr, m->iA, HID, HID, 1);
-  gemm<NTH>(stream, m->iA, HID, 1, p + OFF_W2, HID, 1, n, HID, HID, p + OFF_B2, nullptr, m->iB, HID, HID, 1);
-  gemm<NTH>(stream, m->iB, HID, 1, p + OFF_W3, HID, 1, n, HID, HID, p + OFF_B3, nullptr, m->iA, HID, HID, 1);
-  gemm<1>(stream, m->iA, HID, 1, p + OFF_W4, OUT, 1, n, OUT, HID, p + OFF_B4, nullptr, m->iY, OUT, OUT, 0);
+  gemm<NTH>(stream, m->iX, IN, p + OFF_W1, HID, n, HID, IN, p + OFF_B1, m->iA, HID, 1);
+  gemm<NTH>(stream, m->iA, HID, p + OFF_W2, HID, n, HID, HID, p + OFF_B2, m->iB, HID, 1);
+  gemm<NTH>(stream, m->iB, HID, p + OFF_W3, HID, n, HID, HID, p + OFF_B3, m->iA, HID, 1);
+  gemm<1>(stream, m->iA, HID, p + OFF_W4, OUT, n, OUT, HID, p + OFF_B4, m->iY, OUT, 0);
   hipLaunchKernelGGL(k_denorm, dim3(g1(n)), dim3(256), 0, stream, m->iY, p + OFF_YMU, P, (long)n);
   MCHK(hipGetLastError(), "mlp infer launch");
   MCHK(hipStreamSynchronize(stream), "mlp infer sync");
@@ -824,15 +1015,21 @@ int grad(void* h, const float* X, const float* T, int64_t n, float* loss_out,
          float* grad_host) {
   Net* m = static_cast<Net*>(h);
   if (!m || !X || !T || n <= 0) return mfail(HYQ_EINVAL, "bad argument");
-  int rc = ensure_cap(m, n);
+  const long npad = train_pad(n);
+  int rc = ensure_cap(m, npad);
   if (rc) return rc;
-  MCHK(hipMemsetAsync(m->loss, 0, sizeof(float), m->stream), "loss reset");
-  hipLaunchKernelGGL(k_normalize, dim3(g1(n * 16)), dim3(256), 0, m->stream, X, m->blob + OFF_XMU,
-                     m->Xn, (long)n);
-  forward(m, n);
-  hipLaunchKernelGGL(k_mse_grad, dim3(g1(n)), dim3(256), 0, m->stream, m->Y, T, m->blob + OFF_YMU,
-                     m->dY, (long)n, m->loss);
-  backward(m, n);
+  if (m->tpack_version != m->version) {
+    hipLaunchKernelGGL(k_pack, dim3(g1(PK_N)), dim3(256), 0, m->stream, m->blob, m->tpack);
+    hipLaunchKernelGGL(k_pack_t, dim3(g1(PT_N)), dim3(256), 0, m->stream, m->blob, m->tpack + PK_N);
+    m->tpack_version = m->version;
+  }
+  const int nb = row_blocks(npad), rows = wgrad_rows(npad), nw = wgrad_parts(npad);
+  hipLaunchKernelGGL(k_train_rows, dim3(nb), dim3(64 * kRowWaves), 0, m->stream, X, T, (long)n, npad,
+                     m->blob, m->tpack, m->tpack + PK_N, m->tr, m->bpart);
+  hipLaunchKernelGGL(k_wgrad, dim3(nw, (WT_N + 3) / 4), dim3(256), 0, m->stream, m->tr, npad, rows,
+                     m->wpart);
+  hipLaunchKernelGGL(k_grad_sum, dim3(g1(NPARAM + 1, 64)), dim3(64), 0, m->stream, m->wpart, nw,
+                     m->bpart, nb, m->grad, m->loss);
   MCHK(hipGetLastError(), "mlp grad launch");
   MCHK(hipStreamSynchronize(m->stream), "mlp grad sync");
   if (loss_out) MCHK(hipMemcpy(loss_out, m->loss, sizeof(float), hipMemcpyDeviceToHost), "loss");

@@ -126,6 +126,40 @@ def test_gradient_matches_reference(hidden):
 
 
 @pytest.mark.parametrize("hidden", WIDTHS)
+@pytest.mark.parametrize("n", [1, 31, 33, 4099, 16417, 20001])
+def test_gradient_at_the_edges_of_its_splits(n, hidden):
+    """Batches around the 16- and 32-row tiles, the 256-row parts of the weight gradients (16417
+    rows: 64 parts and a remainder) and one more pass of the row blocks (20001 rows).  The bound
+    is that of test_gradient_matches_reference; a row left out or counted twice in 20001 moves a
+    gradient by less than that, so the targets of the last rows are made to dominate: ten rows
+    with errors 1000 times the others'.  Run twice: the sums have a fixed order."""
+    from hyqmom_amd.warmstart import WarmStartMLP
+    blob = R.random_blob(23, hidden=hidden)
+    rng = np.random.default_rng(24 + n)
+    X = rng.standard_normal((n, 16)).astype(np.float32)
+    T = rng.standard_normal((n, 2)).astype(np.float32) * 0.5
+    T[-10:] *= 1000.0
+    m = WarmStartMLP(blob)
+    Xd, Td = _dev(X), _dev(T)
+    loss, g = m.grad(Xd, Td)
+    lref, gref = R.loss_and_grad(blob, X, T, use_bf16=True)
+    assert abs(loss - lref) <= 1e-3 * lref, (loss, lref)
+    o = 0
+    for name, shp in R.shapes(hidden):
+        k = int(np.prod(shp))
+        a, b = g[o:o + k], gref[o:o + k]
+        o += k
+        nb = np.linalg.norm(b)
+        if nb == 0:
+            assert np.all(a == 0), name
+            continue
+        rel = np.linalg.norm(a - b) / nb
+        assert rel < 1e-2, (n, name, rel)
+    loss2, g2 = m.grad(Xd, Td)
+    assert loss2 == loss and np.array_equal(g, g2)
+
+
+@pytest.mark.parametrize("hidden", WIDTHS)
 def test_training_reduces_loss(hidden):
     """Adam on a smooth synthetic regression: the loss falls by an order of magnitude."""
     import torch
