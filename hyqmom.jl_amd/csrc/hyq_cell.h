@@ -54,7 +54,11 @@ struct ClosureState {
 // standardized moments the closure uses.
 HD S28 standardize28(const double* c, double sx, double sy, double sz) {
   S28 s;
-#define SD(i, j, k) (c[tpos(i, j, k)] / (pw<i>(sx) * pw<j>(sy) * pw<k>(sz)))
+  // 28 quotients by products of powers of sx, sy, sz: the reciprocals of those products start
+  // from the same products of the three reciprocals
+  const double rx = Recip(sx).approx(), ry = Recip(sy).approx(), rz = Recip(sz).approx();
+#define SD(i, j, k) \
+  Recip(pw<i>(sx) * pw<j>(sy) * pw<k>(sz), pw<i>(rx) * pw<j>(ry) * pw<k>(rz)).of(c[tpos(i, j, k)])
   s.S300 = SD(3, 0, 0); s.S400 = SD(4, 0, 0); s.S110 = SD(1, 1, 0); s.S210 = SD(2, 1, 0);
   s.S310 = SD(3, 1, 0); s.S120 = SD(1, 2, 0); s.S220 = SD(2, 2, 0); s.S030 = SD(0, 3, 0);
   s.S130 = SD(1, 3, 0); s.S040 = SD(0, 4, 0); s.S101 = SD(1, 0, 1); s.S201 = SD(2, 0, 1);
@@ -64,6 +68,26 @@ HD S28 standardize28(const double* c, double sx, double sy, double sz) {
   s.S012 = SD(0, 1, 2); s.S112 = SD(1, 1, 2); s.S013 = SD(0, 1, 3); s.S022 = SD(0, 2, 2);
 #undef SD
   return s;
+}
+
+// The edge/corner branch of closure_project (:107-124), kept out of line.
+HYQ_COLD void edge_branch(S28* sp, double R110, double R101, double R011, uint32_t* flp) {
+  S28& s = *sp;
+  uint32_t& fl = *flp;
+  // edge/corner branch (:107-124) with check2D of the three planes (:83-88)
+  fl |= F_EDGE;
+  const P10 p1 = check2D(P10{s.S300, s.S400, s.S110, s.S210, s.S310, s.S120, s.S220, s.S030, s.S130, s.S040}, fl);
+  const P10 p2 = check2D(P10{s.S300, s.S400, s.S101, s.S201, s.S301, s.S102, s.S202, s.S003, s.S103, s.S004}, fl);
+  const P10 p3 = check2D(P10{s.S030, s.S040, s.S011, s.S021, s.S031, s.S012, s.S022, s.S003, s.S013, s.S004}, fl);
+  edge_corner(R110, R101, R011, s, p1, p2, p3);
+  // :107-109: realizable_2D returns (S21, S12, S31, S22, S13), which the xz and yz calls
+  // destructure into (S201, S301, S102, S202, S103) and (S021, S031, S012, S022, S013):
+  // the corrected S102 lands in S301 and S301's in S102 (likewise S012 and S031)
+  realizable_2D(s.S300, s.S400, s.S110, s.S210, s.S310, s.S120, s.S220, s.S030, s.S130, s.S040, fl);
+  realizable_2D(s.S300, s.S400, s.S101, s.S201, s.S301, s.S102, s.S202, s.S003, s.S103, s.S004, fl);
+  { const double t = s.S301; s.S301 = s.S102; s.S102 = t; }
+  realizable_2D(s.S030, s.S040, s.S011, s.S021, s.S031, s.S012, s.S022, s.S003, s.S013, s.S004, fl);
+  { const double t = s.S031; s.S031 = s.S012; s.S012 = t; }
 }
 
 // Flux_closure35_and_realizable_3D (src/numerics/Flux_closure35_and_realizable_3D.jl:33-234),
@@ -94,25 +118,23 @@ HD void closure_project(const double* M4, int flag2D, double Ma, ClosureState& q
 
   const double R110 = 1 - s.S110 * s.S110, R101 = 1 - s.S101 * s.S101, R011 = 1 - s.S011 * s.S011;
   if (R110 <= 0 || R101 <= 0 || R011 <= 0) {
-    // edge/corner branch (:107-124) with check2D of the three planes (:83-88)
-    fl |= F_EDGE;
-    const P10 p1 = check2D(P10{s.S300, s.S400, s.S110, s.S210, s.S310, s.S120, s.S220, s.S030, s.S130, s.S040}, fl);
-    const P10 p2 = check2D(P10{s.S300, s.S400, s.S101, s.S201, s.S301, s.S102, s.S202, s.S003, s.S103, s.S004}, fl);
-    const P10 p3 = check2D(P10{s.S030, s.S040, s.S011, s.S021, s.S031, s.S012, s.S022, s.S003, s.S013, s.S004}, fl);
-    edge_corner(R110, R101, R011, s, p1, p2, p3);
-    // :107-109: realizable_2D returns (S21, S12, S31, S22, S13), which the xz and yz calls
-    // destructure into (S201, S301, S102, S202, S103) and (S021, S031, S012, S022, S013):
-    // the corrected S102 lands in S301 and S301's in S102 (likewise S012 and S031)
-    realizable_2D(s.S300, s.S400, s.S110, s.S210, s.S310, s.S120, s.S220, s.S030, s.S130, s.S040, fl);
-    realizable_2D(s.S300, s.S400, s.S101, s.S201, s.S301, s.S102, s.S202, s.S003, s.S103, s.S004, fl);
-    { const double t = s.S301; s.S301 = s.S102; s.S102 = t; }
-    realizable_2D(s.S030, s.S040, s.S011, s.S021, s.S031, s.S012, s.S022, s.S003, s.S013, s.S004, fl);
-    { const double t = s.S031; s.S031 = s.S012; s.S012 = t; }
+    S28 t = s;
+    uint32_t tf = 0;
+    edge_branch(&t, R110, R101, R011, &tf);
+    s = t;
+    fl |= tf;
   } else {
-    const int f220 = realizable_3D(s, fl);
-    if (f220) {
-      fl |= F_220;
-      for (int it = 0; it < 6; ++it) realizable_3D(s, fl);
+    // once, and six more times where the first pass asks for it (flag220), from one copy of
+    // the code: two inlined copies no longer fit the instruction cache
+    int left = 0;
+    for (bool first = true;; first = false) {
+      const int f220 = realizable_3D(s, fl);
+      if (first) {
+        if (!f220) break;
+        fl |= F_220;
+        left = 6;
+      }
+      if (left-- == 0) break;
     }
   }
   if (flag2D == 1) {

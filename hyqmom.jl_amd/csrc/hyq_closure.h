@@ -238,19 +238,21 @@ HD double realizability_S310(double S110, double S101, double S011, double S300,
       S210 * ((1 - S011 * S011) * S300 + (S011 * S101 - S110) * S210 + (S011 * S110 - S101) * S201);
   const double d11 = 1 - S101 * S101, d12 = S101 * S110 - S011, d22 = 1 - S110 * S110;
   const double dD1 = d11 * d22 - d12 * d12;
+  const Recip rD1(dD1);
   const double V0 = S210 - S110 * S300, V1 = S201 - S101 * S300;
-  const double L1 = (V0 * (d11 * V0 + d12 * V1) + V1 * (d12 * V0 + d22 * V1)) / dD1;
+  const double L1 = rD1.of(V0 * (d11 * V0 + d12 * V1) + V1 * (d12 * V0 + d22 * V1));
   double G310b = H200 - L1;
   if (G310b < 0) G310b = 0.0;
-  const double L2 = quadD2(S110, S101, S011, S210, S120, S111) / dD1;
+  const double L2 = rD1.of(quadD2(S110, S101, S011, S210, S120, S111));
   double G310a = S220 - S110 * S110 - L2 + 1000 * EPS;
   if (G310a < 0 || L2 < 0) G310a = 0.0;
   const double sG = beta * sqrt(G310a * G310b);
-  const double lo = S110 + b310 / dD1 - sG, hi = S110 + b310 / dD1 + sG;
+  const double q310 = rD1.of(b310);
+  const double lo = S110 + q310 - sG, hi = S110 + q310 + sG;
   return S310 <= lo ? lo : (S310 >= hi ? hi : S310);
 }
 // realizability_S310_220 (src/realizability/realizability_S310_220.jl:18-37)
-HD double realizability_S310_220(double S110, double S101, double S011, double S210,
+HYQ_COLD double realizability_S310_220(double S110, double S101, double S011, double S210,
                                  double S120, double S111, double S220) {
   const double d11 = 1 - S101 * S101, d12 = S101 * S110 - S011, d22 = 1 - S110 * S110;
   const double L2 = quadD2(S110, S101, S011, S210, S120, S111) / (d11 * d22 - d12 * d12);
@@ -262,7 +264,8 @@ HD double realizability_S211(double e11, double e22, double e33, double e12, dou
                              double d23, double S211, double beta) {
   const double b = e12 * e13;
   const double sG = beta * sqrt(jmax(0.0, (e11 * e22 - e13 * e13) * (e11 * e33 - e12 * e12)));
-  const double lo = d23 + (b - sG) / e11, hi = d23 + (b + sG) / e11;
+  const Recip r11(e11);
+  const double lo = d23 + r11.of(b - sG), hi = d23 + r11.of(b + sG);
   return S211 <= lo ? lo : (S211 >= hi ? hi : S211);
 }
 
@@ -683,9 +686,24 @@ HD int realizable_3D(S28& s, uint32_t& fl) {
 
   // 4x4 minors (:455-608)
   delta2star(s, E);
-  auto minor4 = [&](const Lead4& L, double Sxx, double& smin, double& smax) {
-    smin = Sxx;
-    smax = Sxx;
+  // the six permutations in one loop: one copy of the cubic solve (six inlined ones were a
+  // third of the projection's code and set its registers)
+  double mn[6], mx[6];
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll 1
+#endif
+  for (int k = 0; k < 6; ++k) {
+    Lead4 L;
+    double Sxx;
+    switch (k) {
+      case 0: L = lead4<0>(E); Sxx = s.S220; break;
+      case 1: L = lead4<2>(E); Sxx = s.S220; break;
+      case 2: L = lead4<1>(E); Sxx = s.S202; break;
+      case 3: L = lead4<3>(E); Sxx = s.S202; break;
+      case 4: L = lead4<4>(E); Sxx = s.S022; break;
+      default: L = lead4<5>(E); Sxx = s.S022;
+    }
+    double smin = Sxx, smax = Sxx;
     if (det4(L) < 0) {
       flag220 = 1;
       fl |= F_R4;
@@ -700,15 +718,17 @@ HD int realizable_3D(S28& s, uint32_t& fl) {
         smax = r3 + d22;
       }
     }
-  };
-  double s220mina, s220maxa, s220minb, s220maxb, s202mina, s202maxa, s202minb, s202maxb,
-      s022mina, s022maxa, s022minb, s022maxb;
-  minor4(lead4<0>(E), s.S220, s220mina, s220maxa);
-  minor4(lead4<2>(E), s.S220, s220minb, s220maxb);
-  minor4(lead4<1>(E), s.S202, s202mina, s202maxa);
-  minor4(lead4<3>(E), s.S202, s202minb, s202maxb);
-  minor4(lead4<4>(E), s.S022, s022mina, s022maxa);
-  minor4(lead4<5>(E), s.S022, s022minb, s022maxb);
+#pragma unroll
+    for (int j = 0; j < 6; ++j)
+      if (j == k) {
+        mn[j] = smin;
+        mx[j] = smax;
+      }
+  }
+  const double s220mina = mn[0], s220minb = mn[1], s202mina = mn[2], s202minb = mn[3],
+               s022mina = mn[4], s022minb = mn[5];
+  const double s220maxa = mx[0], s220maxb = mx[1], s202maxa = mx[2], s202maxb = mx[3],
+               s022maxa = mx[4], s022maxb = mx[5];
   double v;
   v = jmax(jmax(jmax(jmax(jmax(s220mina, s220minb), S220_diag), S220_310), S220_310r), S220_211);
   s.S220 = jmin(jmin(jmin(v, S220max), s220maxa), s220maxb);

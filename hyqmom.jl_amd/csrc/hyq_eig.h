@@ -19,6 +19,28 @@ struct Plane {  // standardized central moments of one plane (c20 = c02 = 1)
   bool ok;        // false if a variance is not positive / not finite
 };
 
+// The plane of central moments cij (i: flux direction) with the flux mean a.
+HD Plane plane_of(double c20, double c11, double c02, double c30, double c21, double c12,
+                  double c03, double c40, double c31, double c22, double c13, double c04, double a) {
+  Plane p;
+  p.a = a;
+  p.ok = (c20 > 0) && (c02 > 0) && (c20 < 1e300) && (c02 < 1e300);
+  const double sf = sqrt(c20), sg = sqrt(c02);
+  p.sig = sf;
+  const double f1 = 1.0 / sf, g1 = 1.0 / sg;
+  const double f2 = f1 * f1, g2 = g1 * g1;
+  p.S11 = c11 * f1 * g1;
+  p.S30 = c30 * f2 * f1;
+  p.S21 = c21 * f2 * g1;
+  p.S12 = c12 * f1 * g2;
+  p.S03 = c03 * g2 * g1;
+  p.S40 = c40 * f2 * f2;
+  p.S31 = c31 * f2 * f1 * g1;
+  p.S22 = c22 * f2 * g2;
+  p.S13 = c13 * f1 * g2 * g1;
+  p.S04 = c04 * g2 * g2;
+  return p;
+}
 // Plane (f, g) from packed central moments c (order <= 4) and the three means.
 template <int F, int G>
 HD Plane plane(const double* c, double um, double vm, double wm) {
@@ -28,25 +50,8 @@ HD Plane plane(const double* c, double um, double vm, double wm) {
     e[G] += j;
     return c[tpos(e[0], e[1], e[2])];
   };
-  Plane p;
-  const double c20 = C(2, 0), c02 = C(0, 2);
-  p.a = F == 0 ? um : (F == 1 ? vm : wm);
-  p.ok = (c20 > 0) && (c02 > 0) && (c20 < 1e300) && (c02 < 1e300);
-  const double sf = sqrt(c20), sg = sqrt(c02);
-  p.sig = sf;
-  const double f1 = 1.0 / sf, g1 = 1.0 / sg;
-  const double f2 = f1 * f1, g2 = g1 * g1;
-  p.S11 = C(1, 1) * f1 * g1;
-  p.S30 = C(3, 0) * f2 * f1;
-  p.S21 = C(2, 1) * f2 * g1;
-  p.S12 = C(1, 2) * f1 * g2;
-  p.S03 = C(0, 3) * g2 * g1;
-  p.S40 = C(4, 0) * f2 * f2;
-  p.S31 = C(3, 1) * f2 * f1 * g1;
-  p.S22 = C(2, 2) * f2 * g2;
-  p.S13 = C(1, 3) * f1 * g2 * g1;
-  p.S04 = C(0, 4) * g2 * g2;
-  return p;
+  return plane_of(C(2, 0), C(1, 1), C(0, 2), C(3, 0), C(2, 1), C(1, 2), C(0, 3), C(4, 0), C(3, 1),
+                  C(2, 2), C(1, 3), C(0, 4), F == 0 ? um : (F == 1 ? vm : wm));
 }
 
 // Standardized flux Jacobian (row-major 6x6).
@@ -89,14 +94,14 @@ HD void balance_n(double* A) {
       for (int j = 0; j < N; ++j)
         if (j != i) { c += fabs(A[j * N + i]); r += fabs(A[i * N + j]); }
       if (c != 0.0 && r != 0.0) {
-        double g = r / 2.0, f = 1.0;
+        // f is a power of two and gi its exact reciprocal: a product with gi is the quotient
+        double g = r / 2.0, f = 1.0, gi = 1.0;
         const double s = c + r;
-        while (c < g) { f *= 2.0; c *= 4.0; }
+        while (c < g) { f *= 2.0; gi *= 0.5; c *= 4.0; }
         g = r * 2.0;
-        while (c > g) { f /= 2.0; c /= 4.0; }
-        if ((c + r) / f < 0.95 * s) {
+        while (c > g) { f *= 0.5; gi *= 2.0; c *= 0.25; }
+        if ((c + r) * gi < 0.95 * s) {
           done = false;
-          const double gi = 1.0 / f;
           for (int j = 0; j < N; ++j) A[i * N + j] *= gi;
           for (int j = 0; j < N; ++j) A[j * N + i] *= f;
         }
@@ -167,10 +172,11 @@ HD void house(double x, double y, double z, bool three, double& v1, double& v2, 
   v2 = three ? z : 0.0;
   if (sig == 0.0) { beta = 0.0; return; }
   const double mu = sqrt(x * x + sig);
-  const double v0 = (x <= 0) ? x - mu : -sig / (x + mu);
-  beta = 2.0 * v0 * v0 / (sig + v0 * v0);
-  v1 = y / v0;
-  v2 = three ? z / v0 : 0.0;
+  const double v0 = (x <= 0) ? x - mu : Recip(x + mu).of(-sig);
+  beta = Recip(sig + v0 * v0).of(2.0 * v0 * v0);
+  const Recip r0(v0);
+  v1 = r0.of(y);
+  v2 = three ? r0.of(z) : 0.0;
 }
 // Francis double-shift QR on an upper Hessenberg matrix, on any 2D accessor H(i, j); each
 // deflated eigenvalue (or conjugate pair) goes to sink(index, re, im).  Returns false if it
@@ -442,12 +448,14 @@ HD EigRes plane_eigs(const Plane& p, uint32_t& fl) {
 // (l-a1)(l-a2)(l-a3) - b2 (l-a3) - b3 (l-a1).  Returns min/max real parts.
 HD void closure1d_speeds(double m0, double m1, double m2, double m3, double m4, double& vmin,
                          double& vmax) {
-  const double a1 = m1 / m0;
+  const Recip r0(m0);
+  const double a1 = r0.of(m1);
   const double s33 = m2 - a1 * m1, s34 = m3 - a1 * m2, s35 = m4 - a1 * m3;
-  const double a2 = s34 / s33 - m1 / m0;
-  const double b2 = s33 / m0;
+  const Recip r33(s33);
+  const double a2 = r33.of(s34) - a1;
+  const double b2 = r0.of(s33);
   const double s44 = s35 - a2 * s34 - b2 * m2;
-  double b3 = s44 / s33;
+  double b3 = r33.of(s44);
   const double a3 = (a1 + a2) / 2;
   b3 = b3 * 5.0 / 2.0;
   if (!(fabs(a1) < 1e300 && fabs(a2) < 1e300 && fabs(b2) < 1e300 && fabs(b3) < 1e300)) {
@@ -458,15 +466,16 @@ HD void closure1d_speeds(double m0, double m1, double m2, double m3, double m4, 
   const double B = -(a1 + a2 + a3);
   const double C = a1 * a2 + a1 * a3 + a2 * a3 - b2 - b3;
   const double D = -a1 * a2 * a3 + b2 * a3 + b3 * a1;
-  const double sh = -B / 3.0;
-  const double p = C - B * B / 3.0;
-  const double q = 2.0 * B * B * B / 27.0 - B * C / 3.0 + D;
-  const double disc = (q / 2.0) * (q / 2.0) + (p / 3.0) * (p / 3.0) * (p / 3.0);
+  const double sh = div3(-B);
+  const double p = C - div3(B * B);
+  const double q = Recip(27.0, 1.0 / 27.0).of(2.0 * B * B * B) - div3(B * C) + D;
+  const double p3 = div3(p);
+  const double disc = (q / 2.0) * (q / 2.0) + p3 * p3 * p3;
   if (disc <= 0.0 && p < 0.0) {  // three real roots (trigonometric form)
-    const double r = 2.0 * sqrt(-p / 3.0);
+    const double r = 2.0 * sqrt(div3(-p));
     double arg = 3.0 * q / (p * r);
     arg = arg > 1.0 ? 1.0 : (arg < -1.0 ? -1.0 : arg);
-    const double th = acos(arg) / 3.0;
+    const double th = div3(acos(arg));
     const double t0 = r * cos(th), t1 = r * cos(th - 2.0943951023931957),
                  t2 = r * cos(th - 4.1887902047863905);
     vmin = sh + fmin(t0, fmin(t1, t2));

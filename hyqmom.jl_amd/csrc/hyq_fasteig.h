@@ -50,11 +50,11 @@ HD int sturm_rem(const double* a, const double* b, double* out) {
   double r[DA + 1];
 #pragma unroll
   for (int t = 0; t <= DA; ++t) r[t] = a[t];
-  const double lb = b[DA - 1];
-  double q = r[DA] / lb;
+  const Recip lb(b[DA - 1]);
+  double q = lb.of(r[DA]);
 #pragma unroll
   for (int t = 0; t < DA; ++t) r[t + 1] -= q * b[t];
-  q = r[DA - 1] / lb;
+  q = lb.of(r[DA - 1]);
 #pragma unroll
   for (int t = 0; t < DA; ++t) r[t] -= q * b[t];
   double m = 0.0;
@@ -62,7 +62,7 @@ HD int sturm_rem(const double* a, const double* b, double* out) {
   for (int t = 0; t <= DA - 2; ++t) m = fmax(m, fabs(r[t]));
   if (!(m > 1e-15)) return 1;
   if (!(m > 1e-9) || !(fabs(r[DA - 2]) > 1e-12 * m)) return 2;
-  const double inv = -1.0 / m;
+  const double inv = Recip(m).of(-1.0);
 #pragma unroll
   for (int t = 0; t <= DA - 2; ++t) out[t] = r[t] * inv;
   return 0;
@@ -169,11 +169,12 @@ HD int laguerre_extreme(const double c[7], double& x, int kmax, bool simple) {
       p = p * x + c[t];
     }
     if (p == 0.0) return it;
-    const double G = dp / p;
-    const double H = G * G - d2p / p;
+    const Recip rp(p);
+    const double G = rp.of(dp);
+    const double H = G * G - rp.of(d2p);
     const double sq = sqrt(fmax((n - 1.0) * (n * H - G * G), 0.0));
     const double den = G >= 0.0 ? G + sq : G - sq;
-    const double dx = n / den;
+    const double dx = Recip(den).of(n);
     x -= dx;
     if (!(fabs(dx) > tol * (1.0 + fabs(x)))) return it;
   }

@@ -2,25 +2,26 @@
 //
 // Device layout: the state is 35 structure-of-arrays moment planes of N = Nx*Ny*Nz
 // doubles, cell index i + Nx*(j + Ny*k) -- the reference's own (Nx,Ny,Nz,35) Julia layout,
-// so host upload/download is a straight copy.  One step is four launches on the context
-// stream, none of which waits on the host:
-//   k_step_begin  : active = (t < tmax); nn += active                      (1 thread)
-//   k_pass1       : per cell: closure -> x/y/z wave speeds -> closure + fluxes -> 1D
-//                   speeds; writes Mr, Fx/Fy/Fz, vp, flags; wave max |vp| -> atomic max
+// so host upload/download is a straight copy.  One step is a chain of launches on the context
+// stream, none of which waits on the host (hyq_step_kernels.h holds the cell kernels):
+//   k_step_begin  : active = (t < tmax); nn += active; the step's counters to 0   (1 thread)
+//   pass 1        : k_project, k_planes (fast modes: k_solve), k_hard, k_close: projection,
+//                   x/y/z wave speeds, closure + fluxes, 1D speeds; writes Mr, Fx/Fy/Fz,
+//                   vp, flags; wave max |vp| -> atomic max
 //   k_dt          : dt = min(CFL*min(dx,dy,dz)/vmax, min(dtmax,Kn), tmax-t); t += dt
 //   k_update      : per cell: x/y/z HLL updates with the reference's boundary rules,
 //                   combined as Mx+My+Mz-2M
-//   k_pass2       : per cell: closure -> x/y wave-speed corrections -> closure -> BGK
+//   pass 2        : k_project, k_planes (k_solve), k_hard, k_relax: projection, x/y wave-speed
+//                   corrections, projection, BGK
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
 #include <cstring>
-#include <mutex>
 #include <string>
 #include <vector>
 
 #include "../../include/hyqmom.h"
-#include "hyq_pipeline.h"
+#include "hyq_step_kernels.h"
 #include "hyq_update.h"
 
 using namespace hyq;
@@ -55,16 +56,6 @@ int fail(int code, const char* what, hipError_t e = hipSuccess) {
   } while (0)
 
 constexpr int kBlock = 128;
-// Minimum waves per SIMD the register allocator must allow for the pass kernels: more waves
-// hide more latency at the price of spills to scratch.  Measured on the 120x120x60 workload,
-// 2 beats 1 for every pass kernel, and the fast kernels are slower at 3 or 4.
-constexpr int kPassWaves = 2, kFastWaves = 2;
-// The fast modes' projection kernels (k_pass1a, k_pass2_relax) need about 310 registers:
-// one wave per SIMD holds them without scratch, where two waves spill 180-190 B per lane;
-// measured 5-15 us faster each at 120x120x60 (k_pass2_check, 196 B of spill at two waves,
-// was 35 us slower at one).
-constexpr int kProjWaves = 1;
-
 constexpr int kNev = 5;  // timing events per step
 constexpr const char* kNonfiniteMsg =
     "non-finite Jacobian in the z wave-speed solve (eigenvalues6z_hyperbolic_3D.jl:108,121 throws)";
@@ -74,54 +65,36 @@ struct DevScalars {  // device-resident step scalars
   unsigned long long vmax_bits;
   long long nn, nnmax;
   unsigned long long err;  // bit 0: a non-finite z Jacobian (where the reference throws)
-  // fast modes, this step: cells on the full pass 1 / pass 2 (nhard), cells with pending
-  // planes (nslot), pending planes (nitem), and cells a pending plane sent to the full path
-  // (ncplx: a complex pair, the eigenvalue correction)
-  unsigned int nhard1, nhard2, nslot1, nslot2, nitem1, nitem2, ncplx1, ncplx2;
+  StepCounts cnt;
 };
 
-// ---- pass 1 -------------------------------------------------------------------------
-__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const unsigned long long w = __shfl_xor(v, o);
-    v = w > v ? w : v;
+// The one run of a context, or a batch (sc null: no step scalars).
+struct Solo {
+  DevScalars* sc;
+  long long N;
+  int flag2D, positivity;
+  double Ma, Kn;
+  __device__ __forceinline__ CellCtx cell() const {
+    CellCtx x;
+    x.active = sc == nullptr || sc->active != 0.0;
+    x.in = false;
+    x.c = 0;
+    x.flag2D = flag2D;
+    x.positivity = positivity;
+    x.Ma = Ma;
+    x.Kn = Kn;
+    x.dt = sc != nullptr ? sc->dt : 0.0;
+    x.vmax = sc != nullptr ? &sc->vmax_bits : nullptr;
+    x.err = sc != nullptr ? &sc->err : nullptr;
+    return x;
   }
-  return v;
-}
-
-template <typename FT, int EM>
-__global__ __launch_bounds__(kBlock, EM == 0 ? kPassWaves : kFastWaves) void k_pass1(const double* __restrict__ M,
-                                                  double* __restrict__ Mr, FT* __restrict__ F,
-                                                  FT* __restrict__ vp, uint32_t* __restrict__ flags,
-                                                  DevScalars* sc, long long N, int flag2D,
-                                                  double Ma, int positivity) {
-  if (sc != nullptr && sc->active == 0.0) return;
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  unsigned long long vb = 0;
-  if (c < N) {
-    double m[35], mr[35], v[6];
-#pragma unroll
-    for (int n = 0; n < 35; ++n) m[n] = M[(size_t)n * N + c];
-    uint32_t fl = 0;
-    pass1_cell<FT, EM>(m, flag2D, Ma, positivity != 0, mr, F + c, F + (size_t)35 * N + c,
-                       F + (size_t)70 * N + c, (size_t)N, v, fl);
-#pragma unroll
-    for (int n = 0; n < 35; ++n) Mr[(size_t)n * N + c] = mr[n];
-#pragma unroll
-    for (int d = 0; d < 6; ++d) {
-      vp[(size_t)d * N + c] = (FT)v[d];
-      const unsigned long long b = __double_as_longlong(fabs(v[d]));
-      vb = b > vb ? b : vb;  // |vp| >= 0: bit order = value order; NaN sorts above +Inf
-    }
-    if (flags) flags[c] = fl;
-    if (sc != nullptr && (fl & F_NONFIN)) atomicOr(&sc->err, 1ull);
+  __device__ __forceinline__ CellCtx cell(unsigned block, int threads, unsigned t) const {
+    CellCtx x = cell();
+    x.c = (long long)block * threads + t;
+    x.in = x.c < N;
+    return x;
   }
-  if (sc != nullptr) {
-    vb = wave_max_u64(vb);
-    if ((threadIdx.x & 63) == 0) atomicMax(&sc->vmax_bits, vb);
-  }
-}
+};
 
 // ---- dt (simulation_runner.jl:402-433, :496) -------------------------------------------
 __global__ void k_step_begin(DevScalars* sc) {
@@ -129,9 +102,7 @@ __global__ void k_step_begin(DevScalars* sc) {
   sc->active = act ? 1.0 : 0.0;
   if (act) sc->nn += 1;
   sc->vmax_bits = 0ull;
-  sc->nhard1 = 0u;
-  sc->nhard2 = 0u;
-  sc->nslot1 = sc->nslot2 = sc->nitem1 = sc->nitem2 = sc->ncplx1 = sc->ncplx2 = 0u;
+  clear_counts(&sc->cnt);
 }
 __global__ void k_dt(DevScalars* sc, double CFL, double hmin, double dtmax, double Kn) {
   if (sc->active == 0.0) return;
@@ -162,23 +133,6 @@ __global__ __launch_bounds__(kUpdBlock) void k_update(const double* __restrict__
   const int k = (int)(c / ((long long)Nx * Ny));
   const double dt = sc->dt;
   update_cell<FT>(Mr, F, vp, Mout, c, i, j, k, Nx, Ny, Nz, N, dt / dx, dt / dy, dt / dz);
-}
-
-// ---- pass 2 + BGK ----------------------------------------------------------------------
-template <bool MIXED, int EM>
-__global__ __launch_bounds__(kBlock, EM == 0 ? kPassWaves : kFastWaves) void k_pass2(double* __restrict__ M, const DevScalars* sc,
-                                                  long long N, int flag2D, double Ma,
-                                                  int positivity, double Kn) {
-  if (sc->active == 0.0) return;
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= N) return;
-  double m[35], o[35];
-#pragma unroll
-  for (int n = 0; n < 35; ++n) m[n] = M[(size_t)n * N + c];
-  uint32_t fl = 0;
-  pass2_cell<MIXED, EM>(m, flag2D, Ma, positivity != 0, sc->dt, Kn, o, fl);
-#pragma unroll
-  for (int n = 0; n < 35; ++n) M[(size_t)n * N + c] = o[n];
 }
 
 // ---- batch kernels ---------------------------------------------------------------------
@@ -372,8 +326,7 @@ __global__ __launch_bounds__(kBlock) void k_plane_dataset(const double* __restri
     }
   }
 }
-// Pass 1, first half: projection (state written to A) and, with FEAT, the network's work.
-// FEAT: a plane whose standardized moments are within kNetTol of a Gaussian's takes the
+// The learned mode's projection (k_project) with the network's work: a plane whose standardized moments are within kNetTol of a Gaussian's takes the
 // Gaussian's extreme eigenvalues, -sqrt(3), +sqrt(3), as its seeds (written to P directly;
 // NaN for a plane that is not finite); the others are handed to the network as compacted
 // rows, normalized with `norm` (16 means, 16 standard deviations) and rounded to bf16 as the
@@ -384,13 +337,11 @@ __global__ __launch_bounds__(kBlock) void k_plane_dataset(const double* __restri
 // seg[wave].  No atomics: the network's kernel reads each segment's count.
 constexpr unsigned kSegRows = 320;  // 64 lanes x 5 planes
 __device__ __forceinline__ short to_bf16(float f) { return __builtin_bit_cast(short, (__bf16)f); }
-template <bool FEAT>
-__global__ __launch_bounds__(kBlock, kProjWaves) void k_pass1a(const double* __restrict__ M, double* __restrict__ A,
-                                                   short* __restrict__ Xb, unsigned* __restrict__ idx,
-                                                   unsigned* __restrict__ seg, float* __restrict__ P,
-                                                   uint32_t* __restrict__ flags, DevScalars* sc,
-                                                   long long N, int flag2D, double Ma,
-                                                   const float* __restrict__ norm) {
+__global__ __launch_bounds__(kBlock, kProjWaves) void k_project_feat(
+    const double* __restrict__ M, double* __restrict__ A, short* __restrict__ Xb,
+    unsigned* __restrict__ idx, unsigned* __restrict__ seg, float* __restrict__ P,
+    uint32_t* __restrict__ flags, DevScalars* sc, long long N, int flag2D, double Ma,
+    const float* __restrict__ norm) {
   if (sc->active == 0.0) return;
   const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= N) return;  // whole waves past N never run; the last wave's lane 0 is inside
@@ -402,7 +353,6 @@ __global__ __launch_bounds__(kBlock, kProjWaves) void k_pass1a(const double* __r
 #pragma unroll
   for (int t = 0; t < 35; ++t) HYQ_STORE_STREAM(&A[(size_t)t * N + c], a[t]);
   flags[c] = fl;
-  if (!FEAT) return;
   Plane pl[5];
   cell_planes(a, pl);
   const unsigned lane = threadIdx.x & 63;
@@ -435,577 +385,6 @@ __global__ __launch_bounds__(kBlock, kProjWaves) void k_pass1a(const double* __r
     used += (unsigned)__popcll(want);
   }
   if (lane == 0) seg[wave] = used;
-}
-
-// Spread of a deferred-cell list of n entries over every wave of the grid: each wave takes
-// `per` consecutive entries (per = ceil(n / waves), at most 64) on its first `per` lanes, and
-// the grid strides by waves * per.  Few cells per wave keep the union of their branch paths,
-// which a wave executes, short; the deferred cells are the rare, branch-heavy ones.
-// LANES lanes per entry (1, or 2: a lane pair that shares one cell's work, see PairSolve).
-template <unsigned LANES = 1>
-struct ListSpread {
-  unsigned n, per, wave, lane, stride;
-  __device__ explicit ListSpread(unsigned n_) : n(n_) {
-    const unsigned waves = gridDim.x * (blockDim.x / 64);
-    per = (n + waves - 1) / waves;
-    per = per < 1 ? 1 : (per > 64 / LANES ? 64 / LANES : per);
-    wave = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
-    lane = (threadIdx.x & 63) / LANES;
-    stride = waves * per;
-  }
-  __device__ bool idle() const { return wave * per >= n; }  // the same for every lane of a wave
-  __device__ unsigned first() const { return wave * per + lane; }
-  __device__ bool mine(unsigned i) const { return lane < per && i < n; }  // same on a pair
-};
-// Waves per SIMD of the list kernels (the full path's stages, the slot solver): their lists
-// are short, so each kernel's time is one wave's latency through its stage, which is
-// shortest with the whole register file (1 wave per SIMD: 256 VGPRs and 256 AGPRs, almost
-// no scratch), not with more waves.  Grid: one wave per SIMD (256 CUs x 4 SIMDs), so that
-// every wave with work runs at once, in 128-thread blocks.
-constexpr int kFullWaves = 1, kSolveWaves = 1;
-constexpr unsigned kListBlocks = 256 * 4 * kFullWaves / 2;
-// Pass 2's slot solver (which fits two waves per SIMD: it needs no extremes) and fix-up
-// kernel, which sorts out the slots (up to a quarter of the cells in the middle of a run),
-// run on a grid of two waves per SIMD, with grid-stride loops over the slots.  (Pass 1's
-// fix-up, which only combines speeds, was slower on this grid: more waves, each with its
-// atomic wave maximum.)
-constexpr unsigned kFixupBlocks = 256 * 4 * kFastWaves / 2;
-
-// ---- the fast step (mixed_newton / mixed_learned modes) ------------------------------------
-// A cell whose planes the fast solve proves hyperbolic finishes in the fast kernel.  A plane
-// the small fast kernel cannot decide (a nearly double eigenvalue, whose pair the 2x2 block
-// test decides, or an inconclusive Sturm chain, which the QR decides) leaves its cell
-// pending: the fast kernel still computes the cell's closure, fluxes and 1D speeds, and
-// stores the projected state and the proven planes' extremes in a slot.  A slot kernel then
-// decides the pending planes, and a fix-up kernel combines the cell's speeds, unless a
-// plane has a complex pair: the eigenvalue correction changes the state, and the cell takes
-// the full path, as do cells whose z path clamps the density or re-projects and cells with
-// a non-finite plane.  Every cell gives the values the full path would: the same functions
-// on the same inputs.  The heavy deciding code stays out of the kernels that every cell
-// runs, which keeps their registers (and spills) down.
-struct FastLists {
-  int* cells;          // [N] cells for the full path
-  int* slot_cell;      // [N] cell of each slot
-  unsigned* slot_mask; // [N] pending planes (bits 0..4)
-  unsigned* slot_bad;  // [N] kSlotBad: a pending plane has a complex pair or is not finite
-  uint32_t* slot_fl;   // [N] the cell's flags
-  double* slot_v;      // [16][N] pass 1: plane extremes (10), 1D speeds (6)
-  double* slot_A;      // [35][N] the projected state the planes come from
-  double* full_S;      // [35][N] the state of each full-path cell between its stages
-  double* full_v;      // [6][N] its x/y/z speeds
-  uint32_t* full_fl;   // [N] its flags
-  unsigned* full_known;  // [N] pass 2: the decisions of its x/y planes on full_S (known_of)
-};
-// A slot whose pending planes include a complex pair or a non-finite plane: slot_bad holds
-// this bit; its low bits hold the decisions the plane solves reached (known_of).
-constexpr unsigned kSlotBad = 0x80000000u;
-// Appends cell c with its projected state A to the full path's list; returns its index.
-__device__ __forceinline__ unsigned new_hard(const FastLists& L, unsigned* count, long long c,
-                                             const double* A, uint32_t fl, long long N) {
-  const unsigned i = atomicAdd(count, 1u);
-  L.cells[i] = (int)c;
-#pragma unroll
-  for (int t = 0; t < 35; ++t) L.full_S[(size_t)t * N + i] = A[t];
-  L.full_fl[i] = fl;
-  return i;
-}
-// Moves slot s (cell c) to the full path's list with the projected state it holds.
-__device__ __forceinline__ unsigned slot_to_hard(const FastLists& L, unsigned* count, unsigned s,
-                                                 long long c, uint32_t fl, long long N) {
-  const unsigned i = atomicAdd(count, 1u);
-  L.cells[i] = (int)c;
-#pragma unroll
-  for (int t = 0; t < 35; ++t) L.full_S[(size_t)t * N + i] = L.slot_A[(size_t)t * N + s];
-  L.full_fl[i] = fl;
-  return i;
-}
-__device__ __forceinline__ unsigned new_slot(const FastLists& L, unsigned* count, long long c,
-                                             unsigned pend, const double* A, long long N) {
-  const unsigned slot = atomicAdd(count, 1u);
-  L.slot_cell[slot] = (int)c;
-  L.slot_mask[slot] = pend;
-  L.slot_bad[slot] = 0u;
-#pragma unroll
-  for (int t = 0; t < 35; ++t) L.slot_A[(size_t)t * N + slot] = A[t];
-  return slot;
-}
-
-// Pass 1 from the projected state that k_pass1a left in AMr (and, in the learned mode, the
-// network's seeds in P).
-// The common cells' wave speeds: the five fast plane solves of the projected state A; a
-// proven cell's six plane extremes (min and max over its two planes per direction) go to
-// vp, for k_pass1_close to combine with the 1D speeds; a cell with pending planes gets a
-// slot, one for the full path a list entry.  The closure and the fluxes of every cell are
-// k_pass1_close's, after the deferred cells: this kernel holds the plane solves' registers
-// only (96 B of scratch per lane at two waves per SIMD, against 568 B with the closure).
-template <typename FT>
-__global__ __launch_bounds__(kBlock, kFastWaves) void k_pass1_fast(
-    const double* __restrict__ A, FT* __restrict__ vp, uint32_t* __restrict__ flags,
-    const float* __restrict__ P, FastLists L, DevScalars* sc, long long N, int positivity) {
-  if (sc->active == 0.0) return;
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= N) return;
-  double a[35];
-#pragma unroll
-  for (int t = 0; t < 35; ++t) a[t] = A[(size_t)t * N + c];
-  const uint32_t fl0 = flags[c];
-  uint32_t fl = fl0;
-  Warm w = no_warm();
-  if (P != nullptr) {
-#pragma unroll
-    for (int q = 0; q < 5; ++q) {
-      w.w[2 * q] = P[((size_t)q * N + c) * 2];
-      w.w[2 * q + 1] = P[((size_t)q * N + c) * 2 + 1];
-    }
-  }
-  double v[10];
-  unsigned pend;
-  const int st = fast_cell_planes<false, true>(a, positivity != 0, w, v, pend, fl);
-  if (st == kPlaneFull) {
-    new_hard(L, &sc->nhard1, c, a, fl0, N);  // the full path starts from the projection
-    return;
-  }
-  if (st == kPlaneSolve) {
-    const unsigned slot = new_slot(L, &sc->nslot1, c, pend, a, N);
-    L.slot_fl[slot] = fl;
-#pragma unroll
-    for (int t = 0; t < 10; ++t) L.slot_v[(size_t)t * N + slot] = v[t];
-    return;
-  }
-  double v6[6];
-  combine_planes(v, v6);
-#pragma unroll
-  for (int d = 0; d < 6; ++d) vp[(size_t)d * N + c] = (FT)v6[d];
-  flags[c] = fl;
-}
-
-// Pass 1's closure and fluxes of every cell, after the deferred cells: A (the projected
-// state, or the full path's final state) to its closure Mr in place, the fluxes, the 1D
-// speeds of Mr combined with the plane extremes the speed kernels left in vp (min and max
-// commute with rounding to FT, so combining the rounded extremes gives the same FT speeds),
-// the flags, the wave maximum |vp|.  One wave per SIMD: the closure with fluxes needs about
-// 400 registers.
-template <typename FT>
-__global__ __launch_bounds__(kBlock, kProjWaves) void k_pass1_close(
-    double* __restrict__ AMr, FT* __restrict__ F, FT* __restrict__ vp, uint32_t* __restrict__ flags,
-    DevScalars* sc, long long N, int flag2D, double Ma) {
-  if (sc->active == 0.0) return;
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  unsigned long long vb = 0;
-  if (c < N) {
-    double a[35], mr[35], s1[6], v6[6], vd[6];
-#pragma unroll
-    for (int t = 0; t < 35; ++t) a[t] = HYQ_LOAD_STREAM(&AMr[(size_t)t * N + c]);
-    uint32_t fl = flags[c];
-    flux_closure35<true, FT>(a, flag2D, Ma, mr, F + c, F + (size_t)35 * N + c,
-                             F + (size_t)70 * N + c, (size_t)N, fl);
-    closure1d_all(mr, s1);
-#pragma unroll
-    for (int d = 0; d < 6; ++d) v6[d] = (double)vp[(size_t)d * N + c];
-    combine_vp(s1, v6, vd);
-#pragma unroll
-    for (int d = 0; d < 6; ++d) {
-      vp[(size_t)d * N + c] = (FT)vd[d];
-      const unsigned long long bb = __double_as_longlong(fabs(vd[d]));
-      vb = bb > vb ? bb : vb;
-    }
-#pragma unroll
-    for (int t = 0; t < 35; ++t) HYQ_STORE_STREAM(&AMr[(size_t)t * N + c], mr[t]);
-    flags[c] = fl;
-    if (fl & F_NONFIN) atomicOr(&sc->err, 1ull);
-  }
-  vb = wave_max_u64(vb);
-  if ((threadIdx.x & 63) == 0) atomicMax(&sc->vmax_bits, vb);
-}
-
-// The pending planes of every slot: the fast solve with the 2x2 block test of a nearly double
-// pair, the QR where that does not decide.  One item per (slot, plane), items spread over
-// every wave of the grid (ListSpread), one plane per lane: the kernel's time is one plane
-// solve's latency, not that of a cell's pending planes in turn.  A plane's results go to
-// the slot: its extremes to slot_v (pass 1), its flags and iterations to slot_fl by atomic
-// OR and add (the iteration field, bits 16-27, holds at most 5 x 2 x 40 per pass and the
-// fast kernel's as many, far below its 4095 cap), its decision (known_of) to slot_bad, whose
-// kSlotBad bit marks a complex pair or a non-finite plane.  VALS: pass 1 (extremes; P: the
-// network's seeds or null); pass 2 only needs the decisions.
-template <bool VALS>
-__global__ __launch_bounds__(kBlock, kSolveWaves) void k_slot_solve(FastLists L, const unsigned* count,
-                                                                    unsigned* nplanes,
-                                                                    const float* __restrict__ P,
-                                                                    DevScalars* sc, long long N) {
-  if (sc->active == 0.0) return;
-  constexpr unsigned NP = VALS ? 5u : 4u;  // planes per slot: pass 2 checks x and y only
-  const ListSpread<> ls(*count * NP);
-  if (ls.idle()) return;
-  for (unsigned i = ls.first(); i < ls.n; i += ls.stride) {
-    if (!ls.mine(i)) continue;
-    const unsigned s = i / NP, q = i % NP;
-    const unsigned pend = L.slot_mask[s];
-    if (q == 0) atomicAdd(nplanes, (unsigned)__popc(pend));
-    if (!(pend & (1u << q))) continue;
-    double A[35];
-#pragma unroll
-    for (int t = 0; t < 35; ++t) A[t] = L.slot_A[(size_t)t * N + s];
-    float wmin = NAN, wmax = NAN;
-    if (VALS && P != nullptr) {
-      const long long c = L.slot_cell[s];
-      wmin = P[((size_t)q * N + c) * 2];
-      wmax = P[((size_t)q * N + c) * 2 + 1];
-    }
-    uint32_t fl = 0;
-    double v0 = 0.0, v1 = 0.0;
-    const unsigned d = solve_plane(A, (int)q, VALS, wmin, wmax, v0, v1, fl);
-    if (d != kKnownReal) {
-      atomicOr(&L.slot_bad[s], kSlotBad | (d << (2 * q)));
-      continue;
-    }
-    if (NP == 4) atomicOr(&L.slot_bad[s], d << (2 * q));  // pass 2: the decision for the full path
-    if (VALS) {
-      L.slot_v[(size_t)(2 * q) * N + s] = v0;
-      L.slot_v[(size_t)(2 * q + 1) * N + s] = v1;
-      atomicOr(&L.slot_fl[s], fl & 0xFFFFu);
-      atomicAdd(&L.slot_fl[s], fl & 0xFFFF0000u);
-    }
-  }
-}
-
-// Pass 1 of the cells with plane solves: their speeds, or the full path after a complex pair.
-template <typename FT>
-__global__ __launch_bounds__(kBlock) void k_pass1_fixup(FastLists L, FT* __restrict__ vp,
-                                                        uint32_t* __restrict__ flags, DevScalars* sc,
-                                                        long long N) {
-  if (sc->active == 0.0) return;
-  const unsigned n = sc->nslot1;
-  for (unsigned s = blockIdx.x * blockDim.x + threadIdx.x; s < n; s += gridDim.x * blockDim.x) {
-    const long long c = L.slot_cell[s];
-    if (L.slot_bad[s] & kSlotBad) {
-      atomicAdd(&sc->ncplx1, 1u);
-      slot_to_hard(L, &sc->nhard1, s, c, flags[c], N);  // flags[c]: those of the projection
-      continue;
-    }
-    double v[10], v6[6];
-#pragma unroll
-    for (int t = 0; t < 10; ++t) v[t] = L.slot_v[(size_t)t * N + s];
-    combine_planes(v, v6);
-#pragma unroll
-    for (int d = 0; d < 6; ++d) vp[(size_t)d * N + c] = (FT)v6[d];
-    flags[c] = L.slot_fl[s];
-  }
-}
-
-// The full pass 1 of the listed cells, in stages: x, y and z wave speeds (with their
-// eigenvalue corrections, the z density clamp and re-projection) of the projected state; the
-// closure with the fluxes is k_pass1_close's, with every other cell.  Each stage is one
-// kernel over the list, the cell's state kept in full_S between stages: the same functions,
-// on the same values, as pass1_cell, so the results are the same bits, but each kernel
-// holds one stage's registers instead of the whole path's, which keeps its latency (the
-// kernel's time on a short list) down.  P: the network's seeds (learned mode) or null.
-__device__ __forceinline__ Warm list_warm(const float* P, long long c, long long N) {
-  Warm w = no_warm();
-  if (P != nullptr) {
-#pragma unroll
-    for (int q = 0; q < 5; ++q) {
-      w.w[2 * q] = P[((size_t)q * N + c) * 2];
-      w.w[2 * q + 1] = P[((size_t)q * N + c) * 2 + 1];
-    }
-  }
-  return w;
-}
-// ---- lane pairs: the two plane solves of an axis side by side -------------------------------
-// A full-path cell's stage is a chain of latencies (one wave per SIMD, a few cells per
-// wave), and each axis solves its two planes one after the other.  In pass 1's stage
-// kernels a lane pair shares a cell: both lanes hold the same state and run the same code, except
-// that lane `half` = 0 solves the axis's first plane and lane 1 its second, and the two
-// exchange their results (and the flags their solves set) by a lane swap.  The values, the
-// decisions and the flags are those of eig6_axis / eig6_z: the same plane_solve on the same
-// planes, the flags OR-ed, the root-polishing iterations added (the field cannot reach its
-// 4095 cap: at most 5 planes x 2 solves x 80 per pass, and as many in the fast kernel).
-__device__ __forceinline__ EigRes swap_res(const EigRes& r) {
-  EigRes o;
-  o.vmin = __shfl_xor(r.vmin, 1);
-  o.vmax = __shfl_xor(r.vmax, 1);
-  o.cplx = __shfl_xor((int)r.cplx, 1) != 0;
-  o.ok = __shfl_xor((int)r.ok, 1) != 0;
-  return o;
-}
-HD uint32_t merge_flags(uint32_t fl, uint32_t fa, uint32_t fb) {
-  const uint32_t it = (fl >> 16) + (fa >> 16) + (fb >> 16);
-  return ((fl | fa | fb) & 0xFFFFu) | ((it < 0xFFFu ? it : 0xFFFu) << 16);
-}
-// Planes a and b solved on the two lanes of a pair; A, B: both results on both lanes.
-template <bool CORRECTS>
-__device__ __forceinline__ void pair_solve(const Plane& pa, const Plane& pb, float wa0, float wa1,
-                                           float wb0, float wb1, bool need_vals, uint32_t& fl,
-                                           int half, EigRes& A, EigRes& B) {
-  uint32_t f = 0;
-  const EigRes r = plane_solve<1, CORRECTS>(half ? pb : pa, half ? wb0 : wa0, half ? wb1 : wa1,
-                                            need_vals, f);
-  const EigRes o = swap_res(r);
-  const uint32_t fo = (uint32_t)__shfl_xor((int)f, 1);
-  A = half ? o : r;
-  B = half ? r : o;
-  fl = merge_flags(fl, half ? fo : f, half ? f : fo);
-}
-// eig6_axis<AXIS, 1> on a lane pair.
-template <int AXIS>
-__device__ bool eig6_axis_pair(const double* M, int flag2D, double Ma, double& vmin, double& vmax,
-                               double* Mr, uint32_t& fl, const Warm& wm_, bool need_vals, int half) {
-  double c[35];
-  double M000, um, vm, wm;
-  raw_to_central4(M, c, M000, um, vm, wm);
-  const int ia = AXIS == 0 ? 0 : 2, ib = AXIS == 0 ? 1 : 3;  // Warm slots: UV UW VU VW WU
-  EigRes A, B;
-  pair_solve<true>(AXIS == 0 ? plane<0, 1>(c, um, vm, wm) : plane<1, 0>(c, um, vm, wm),
-                   AXIS == 0 ? plane<0, 2>(c, um, vm, wm) : plane<1, 2>(c, um, vm, wm),
-                   wm_.w[2 * ia], wm_.w[2 * ia + 1], wm_.w[2 * ib], wm_.w[2 * ib + 1], need_vals, fl,
-                   half, A, B);
-  combine_guarded(A, B, vmin, vmax);
-  if (A.cplx || B.cplx) {
-    axis_correct<AXIS>(c, M000, um, vm, wm, A.cplx, B.cplx, flag2D, Ma, Mr, fl);
-    if (!need_vals) return true;
-    raw_to_central4(Mr, c, M000, um, vm, wm);
-    pair_solve<false>(AXIS == 0 ? plane<0, 1>(c, um, vm, wm) : plane<1, 0>(c, um, vm, wm),
-                      AXIS == 0 ? plane<0, 2>(c, um, vm, wm) : plane<1, 2>(c, um, vm, wm),
-                      wm_.w[2 * ia], wm_.w[2 * ia + 1], wm_.w[2 * ib], wm_.w[2 * ib + 1], need_vals,
-                      fl, half, A, B);
-    combine_guarded(A, B, vmin, vmax);
-    return true;
-  }
-#pragma unroll
-  for (int n = 0; n < 35; ++n) Mr[n] = M[n];
-  return false;
-}
-// eig6_z<1> on a lane pair: the density clamp and the re-projection on both lanes, the WU
-// and VW solves side by side.
-__device__ void eig6_z_pair(const double* M, int flag2D, double Ma, bool positivity, double& vmin,
-                            double& vmax, double* Mr, uint32_t& fl, const Warm& wm_, int half) {
-#pragma unroll
-  for (int n = 0; n < 35; ++n) Mr[n] = M[n];
-  if (positivity && M[0] <= 0.0) {
-    Mr[0] = jmax(M[0], 1e-14);
-    fl |= F_RHO;
-  }
-  double W[35];
-#pragma unroll
-  for (int n = 0; n < 35; ++n) W[n] = M[n];
-  W[0] = Mr[0];
-  if (positivity && W[0] > 1e-15) {
-    const double m0 = W[0];
-    const double vx = M[2] / m0 - (M[1] / m0) * (M[1] / m0);
-    const double vy = M[9] / m0 - (M[5] / m0) * (M[5] / m0);
-    const double vz = M[19] / m0 - (M[15] / m0) * (M[15] / m0);
-    if (vx < 0.0 || vy < 0.0 || vz < 0.0) {
-      fl |= F_ZNEG;
-      flux_closure35<false, double>(M, flag2D, Ma, Mr, nullptr, nullptr, nullptr, 0, fl);
-#pragma unroll
-      for (int n = 0; n < 35; ++n) W[n] = Mr[n];
-    }
-  }
-  double c[35];
-  double M000, um, vm, wm;
-  raw_to_central4(W, c, M000, um, vm, wm);
-  EigRes A, B;
-  pair_solve<true>(plane<2, 0>(c, um, vm, wm), plane<1, 2>(c, um, vm, wm), wm_.w[8], wm_.w[9],
-                   wm_.w[6], wm_.w[7], true, fl, half, A, B);
-  if (!A.ok || !B.ok) fl |= F_NONFIN;  // the reference's eigvals throws here
-  vmin = jmin(A.vmin, B.vmin);
-  vmax = jmax(A.vmax, B.vmax);
-  if (A.cplx || B.cplx) {
-    fl |= F_ECZ;
-    raw_to_central4(M, c, M000, um, vm, wm);  // corrections start from the input M
-    double cn[35];
-#pragma unroll
-    for (int t = 0; t < 35; ++t) cn[t] = c[t];
-    if (A.cplx) correct_plane<0, 2>(c, cn);
-    if (B.cplx) correct_plane<1, 2>(c, cn);
-    central_to_raw<4>(cn, M000, um, vm, wm);
-    double Mh[35];
-    pack35(cn, Mh);
-    flux_closure35<false, double>(Mh, flag2D, Ma, Mr, nullptr, nullptr, nullptr, 0, fl);
-    raw_to_central4(Mr, c, M000, um, vm, wm);
-    pair_solve<false>(plane<2, 0>(c, um, vm, wm), plane<1, 2>(c, um, vm, wm), wm_.w[8], wm_.w[9],
-                      wm_.w[6], wm_.w[7], true, fl, half, A, B);
-    vmin = jmin(A.vmin, B.vmin);
-    vmax = jmax(A.vmax, B.vmax);
-  }
-}
-// The list holds each cell's projected state (pass1a_cell, computed once by k_pass1a) and
-// the flags of that projection.  STAGE 1: x; 2: y; 3: z.
-template <int STAGE, typename FT>
-__global__ __launch_bounds__(kBlock, kFullWaves) void k_full1_stage(
-    const float* __restrict__ P, FastLists L, DevScalars* sc, long long N, int flag2D, double Ma,
-    int positivity, double* __restrict__ AMr, FT* __restrict__ vp, uint32_t* __restrict__ flags) {
-  if (sc->active == 0.0) return;
-  const ListSpread<2> ls(sc->nhard1);  // a lane pair per cell
-  if (ls.idle()) return;  // wave-uniform
-  const int half = threadIdx.x & 1;
-  for (unsigned i = ls.first(); i < ls.n; i += ls.stride) {
-    if (!ls.mine(i)) continue;
-    const long long c = L.cells[i];
-    double a[35], b[35];
-#pragma unroll
-    for (int t = 0; t < 35; ++t) a[t] = L.full_S[(size_t)t * N + i];
-    uint32_t fl = L.full_fl[i];
-    const Warm w = list_warm(P, c, N);
-    double mn, mx;
-    if (STAGE == 1) eig6_axis_pair<0>(a, flag2D, Ma, mn, mx, b, fl, w, true, half);
-    if (STAGE == 2) eig6_axis_pair<1>(a, flag2D, Ma, mn, mx, b, fl, w, true, half);
-    if (STAGE == 3) eig6_z_pair(a, flag2D, Ma, positivity != 0, mn, mx, b, fl, w, half);
-    if (half) continue;  // both lanes hold the same results
-    if (STAGE < 3) {
-      L.full_v[(size_t)(2 * (STAGE - 1)) * N + i] = mn;
-      L.full_v[(size_t)(2 * (STAGE - 1) + 1) * N + i] = mx;
-#pragma unroll
-      for (int t = 0; t < 35; ++t) L.full_S[(size_t)t * N + i] = b[t];
-      L.full_fl[i] = fl;
-      continue;
-    }
-    // the cell's final state, speeds and flags, where k_pass1_close takes every cell's
-#pragma unroll
-    for (int d = 0; d < 4; ++d) vp[(size_t)d * N + c] = (FT)L.full_v[(size_t)d * N + i];
-    vp[(size_t)4 * N + c] = (FT)mn;
-    vp[(size_t)5 * N + c] = (FT)mx;
-#pragma unroll
-    for (int t = 0; t < 35; ++t) AMr[(size_t)t * N + c] = b[t];
-    flags[c] = fl;
-  }
-}
-// The full pass 1's stages on `stream`, then the closure and fluxes of every cell.
-template <typename FT>
-static void enqueue_full1(hipStream_t stream, double* AMr, FT* F, FT* vp, uint32_t* flags,
-                          const float* P, const FastLists& L, DevScalars* sc, long long N,
-                          int flag2D, double Ma, int positivity) {
-  hipLaunchKernelGGL((k_full1_stage<1, FT>), dim3(kListBlocks), dim3(kBlock), 0, stream, P, L, sc, N,
-                     flag2D, Ma, positivity, AMr, vp, flags);
-  hipLaunchKernelGGL((k_full1_stage<2, FT>), dim3(kListBlocks), dim3(kBlock), 0, stream, P, L, sc, N,
-                     flag2D, Ma, positivity, AMr, vp, flags);
-  hipLaunchKernelGGL((k_full1_stage<3, FT>), dim3(kListBlocks), dim3(kBlock), 0, stream, P, L, sc, N,
-                     flag2D, Ma, positivity, AMr, vp, flags);
-  hipLaunchKernelGGL(k_pass1_close<FT>, dim3((unsigned)((N + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                     stream, AMr, F, vp, flags, sc, N, flag2D, Ma);
-}
-
-// The fast modes' pass 2: projection and the x/y hyperbolicity checks (projected state to
-// A; A[0] = NaN marks a cell that k_pass2_relax leaves alone), the plane solves, the fix-up
-// of the cells with plane solves (those proven hyperbolic back into A, the others to the
-// full path), BGK of every proven cell, and the full pass 2 of the rest.
-__global__ __launch_bounds__(kBlock, kFastWaves) void k_pass2_check(const double* __restrict__ M,
-                                                                   double* __restrict__ A,
-                                                                   FastLists L, DevScalars* sc,
-                                                                   long long N, int flag2D,
-                                                                   double Ma) {
-  if (sc->active == 0.0) return;
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= N) return;
-  double m[35], a[35];
-#pragma unroll
-  for (int n = 0; n < 35; ++n) m[n] = HYQ_LOAD_STREAM(&M[(size_t)n * N + c]);
-  uint32_t fl = 0;
-  unsigned pend, known;
-  const int st = pass2_check_planes<false>(m, flag2D, Ma, a, pend, fl, &known);
-  if (st == kPlaneProven) {
-#pragma unroll
-    for (int n = 0; n < 35; ++n) HYQ_STORE_STREAM(&A[(size_t)n * N + c], a[n]);
-    return;
-  }
-  A[c] = NAN;
-  if (st == kPlaneFull)
-    L.full_known[new_hard(L, &sc->nhard2, c, a, 0u, N)] = known;
-  else
-    new_slot(L, &sc->nslot2, c, pend, a, N);
-}
-
-__global__ __launch_bounds__(kBlock, kProjWaves) void k_pass2_relax(double* __restrict__ M,
-                                                                   const double* __restrict__ A,
-                                                                   DevScalars* sc, long long N,
-                                                                   int flag2D, double Ma,
-                                                                   int positivity, double Kn) {
-  if (sc->active == 0.0) return;
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= N) return;
-  const double a0 = A[c];
-  if (a0 != a0) return;
-  double a[35], o[35];
-  a[0] = a0;
-#pragma unroll
-  for (int n = 1; n < 35; ++n) a[n] = A[(size_t)n * N + c];
-  uint32_t fl = 0;
-  pass2_relax<true>(a, flag2D, Ma, positivity != 0, sc->dt, Kn, o, fl);
-#pragma unroll
-  for (int n = 0; n < 35; ++n) M[(size_t)n * N + c] = o[n];
-}
-
-// Pass 2 of the cells with plane solves: back into A for k_pass2_relax, or the full path
-// after a complex pair.
-__global__ __launch_bounds__(kBlock, kFastWaves) void k_pass2_fixup(double* __restrict__ A,
-                                                                   FastLists L, DevScalars* sc,
-                                                                   long long N) {
-  if (sc->active == 0.0) return;
-  const unsigned n = sc->nslot2;
-  for (unsigned s = blockIdx.x * blockDim.x + threadIdx.x; s < n; s += gridDim.x * blockDim.x) {
-    const long long c = L.slot_cell[s];
-    const unsigned bad = L.slot_bad[s];
-    if (bad & kSlotBad) {
-      atomicAdd(&sc->ncplx2, 1u);
-      const unsigned i = slot_to_hard(L, &sc->nhard2, s, c, 0u, N);
-      // the planes that were not pending were proven hyperbolic by the check
-      unsigned known = bad & 0xFFu;
-      const unsigned pend = L.slot_mask[s];
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        if (!(pend & (1u << q))) known |= kKnownReal << (2 * q);
-      L.full_known[i] = known;
-      continue;
-    }
-    // proven hyperbolic: back into the relaxation kernel's input A, which then relaxes it
-    // with the cells the check proved
-#pragma unroll
-    for (int t = 0; t < 35; ++t) A[(size_t)t * N + c] = L.slot_A[(size_t)t * N + s];
-  }
-}
-
-// The full pass 2 of the listed cells, in stages like the full pass 1: the x and y
-// corrections of the projected state the check left in the list (with the plane decisions the
-// check and the plane solves reached on it).  Stage 2 hands the corrected state to
-// k_pass2_relax through A, which relaxes it with every other cell (the same BGK on the same
-// state); a state whose density is not a number, which would read as A's "not proven"
-// mark, is relaxed here instead.  STAGE 1: x; 2: y.
-template <int STAGE>
-__global__ __launch_bounds__(kBlock, kFullWaves) void k_full2_stage(FastLists L, DevScalars* sc,
-                                                                   long long N, int flag2D,
-                                                                   double Ma, double* __restrict__ A,
-                                                                   double* __restrict__ M,
-                                                                   int positivity, double Kn) {
-  if (sc->active == 0.0) return;
-  const ListSpread<> ls(sc->nhard2);
-  if (ls.idle()) return;
-  for (unsigned i = ls.first(); i < ls.n; i += ls.stride) {
-    if (!ls.mine(i)) continue;
-    double a[35], b[35];
-    uint32_t fl = 0;
-#pragma unroll
-    for (int t = 0; t < 35; ++t) a[t] = L.full_S[(size_t)t * N + i];
-    const unsigned known = L.full_known[i];
-    // the wave speeds of pass 2 are not used, only its corrections; after an x correction
-    // the y decisions no longer hold
-    const bool corrected = STAGE == 1 ? eig6_axis_decided<0>(a, flag2D, Ma, b, fl, known)
-                                      : eig6_axis_decided<1>(a, flag2D, Ma, b, fl, known);
-    if (STAGE == 1) {
-      if (corrected) L.full_known[i] = known & 0x0Fu;
-#pragma unroll
-      for (int t = 0; t < 35; ++t) L.full_S[(size_t)t * N + i] = b[t];
-      continue;
-    }
-    const long long c = L.cells[i];
-    if (b[0] == b[0]) {
-#pragma unroll
-      for (int t = 0; t < 35; ++t) A[(size_t)t * N + c] = b[t];
-    } else {
-      double o[35];
-      pass2_relax<true>(b, flag2D, Ma, positivity != 0, sc->dt, Kn, o, fl);
-#pragma unroll
-      for (int t = 0; t < 35; ++t) M[(size_t)t * N + c] = o[t];
-    }
-  }
 }
 
 // ---- snapshot fields ----------------------------------------------------------------
@@ -1187,7 +566,7 @@ struct hyq_ctx {
   unsigned* Xidx;  // [segments x kSegRows] plane index q N + c of each row
   unsigned* Xseg;  // [ceil(N / 64)] rows in each wave's segment
   float* P;        // [5N][2] seeds of each plane: the network's predictions or the Gaussian's
-  FastLists L;             // fast modes: full-path list, slots and plane items
+  Lists L;         // the entries of a pass, in F, which is free then
   double* diag;            // [8] results of the diagnostics
 };
 
@@ -1236,20 +615,7 @@ int hyq_create(const hyq_params* params, hyq_ctx** out) {
          // reads counts of 0 (it runs, as every kernel of the step, also in a step that has
          // nothing left to do)
          hipMemset(c->Xseg, 0, sizeof(unsigned) * ((c->N + 63) / 64)) == hipSuccess;
-  if (ok && (params->precision == HYQ_PREC_MIXED_NEWTON || params->precision == HYQ_PREC_MIXED_LEARNED)) {
-    FastLists& L = c->L;
-    ok = hipMalloc(&L.cells, sizeof(int) * c->N) == hipSuccess &&
-         hipMalloc(&L.slot_cell, sizeof(int) * c->N) == hipSuccess &&
-         hipMalloc(&L.slot_mask, sizeof(unsigned) * c->N) == hipSuccess &&
-         hipMalloc(&L.slot_bad, sizeof(unsigned) * c->N) == hipSuccess &&
-         hipMalloc(&L.slot_fl, sizeof(uint32_t) * c->N) == hipSuccess &&
-         hipMalloc(&L.slot_v, sizeof(double) * 16 * c->N) == hipSuccess &&
-         hipMalloc(&L.slot_A, sizeof(double) * 35 * c->N) == hipSuccess &&
-         hipMalloc(&L.full_S, sizeof(double) * 35 * c->N) == hipSuccess &&
-         hipMalloc(&L.full_v, sizeof(double) * 6 * c->N) == hipSuccess &&
-         hipMalloc(&L.full_fl, sizeof(uint32_t) * c->N) == hipSuccess &&
-         hipMalloc(&L.full_known, sizeof(unsigned) * c->N) == hipSuccess;
-  }
+  if (ok) c->L = carve_lists(c->F, c->N);
   if (!ok) {
     hyq_destroy(c);
     return fail(HYQ_ENOMEM, "device allocation failed");
@@ -1278,17 +644,6 @@ int hyq_destroy(hyq_ctx* c) {
   hipFree(c->Xidx);
   hipFree(c->Xseg);
   hipFree(c->P);
-  hipFree(c->L.cells);
-  hipFree(c->L.slot_cell);
-  hipFree(c->L.slot_bad);
-  hipFree(c->L.slot_fl);
-  hipFree(c->L.slot_v);
-  hipFree(c->L.slot_mask);
-  hipFree(c->L.slot_A);
-  hipFree(c->L.full_S);
-  hipFree(c->L.full_v);
-  hipFree(c->L.full_fl);
-  hipFree(c->L.full_known);
   for (int i = 0; i < kNev * kChunk; ++i)
     if (c->ev[i]) hipEventDestroy(c->ev[i]);
   if (c->stream) hipStreamDestroy(c->stream);
@@ -1312,88 +667,64 @@ int hyq_get_state(hyq_ctx* c, double* M) {
   return HYQ_OK;
 }
 
-// One step on the context stream; ev (or null): kNev events bracketing its parts.
-static int enqueue_step(hyq_ctx* c, hipEvent_t* ev) {
+}  // extern "C"
+
+// One step on the context stream; ev (or null): kNev events bracketing its parts.  FT: the
+// fluxes' and speeds' type (float: the mixed modes); EM: 1 for the fast modes.
+template <typename FT, int EM>
+static int enqueue_step_t(hyq_ctx* c, hipEvent_t* ev) {
+  constexpr bool kMixed = sizeof(FT) == 4;
   const hyq_params& p = c->p;
-  const unsigned g = grid_for(c->N);
+  const unsigned g = grid_for(c->N), g64 = (unsigned)((c->N + 63) / 64);
   const double hmin = jmin(jmin(c->dx, c->dy), c->dz);
+  const Solo R{c->sc, c->N, p.flag2D, p.positivity, p.Ma, p.Kn};
+  FT* F = (FT*)c->F;
+  FT* vp = (FT*)c->vp;
   hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(1), 0, c->stream, c->sc);
   if (ev) hipEventRecord(ev[0], c->stream);
-  const bool fast = p.precision == HYQ_PREC_MIXED_NEWTON || p.precision == HYQ_PREC_MIXED_LEARNED;
-  if (p.precision == HYQ_PREC_FP64) {
-    hipLaunchKernelGGL((k_pass1<double, 0>), dim3(g), dim3(kBlock), 0, c->stream, c->M, c->Mr,
-                       (double*)c->F, (double*)c->vp, c->flags, c->sc, c->N, p.flag2D, p.Ma,
-                       p.positivity);
-  } else if (p.precision == HYQ_PREC_MIXED) {
-    hipLaunchKernelGGL((k_pass1<float, 0>), dim3(g), dim3(kBlock), 0, c->stream, c->M, c->Mr,
-                       (float*)c->F, (float*)c->vp, c->flags, c->sc, c->N, p.flag2D, p.Ma,
-                       p.positivity);
+  const bool learned = p.precision == HYQ_PREC_MIXED_LEARNED && c->mlp != nullptr;
+  if (learned) {
+    // the network's input rows and warm starts with the projection
+    hipLaunchKernelGGL(k_project_feat, dim3(g), dim3(kBlock), 0, c->stream, c->M, c->Mr,
+                       reinterpret_cast<short*>(c->X), c->Xidx, c->Xseg, c->P, c->flags, c->sc,
+                       c->N, p.flag2D, p.Ma, hyq_mlp_input_norm(c->mlp));
+    const int rc = hyq_mlp_infer_bf16_segments_async(
+        c->mlp, reinterpret_cast<const short*>(c->X), c->Xidx, c->Xseg, (c->N + 63) / 64,
+        (int32_t)kSegRows, c->P, c->stream);
+    if (rc) return rc;
   } else {
-    // fast modes: projection (+ the network's input rows and warm starts in the learned
-    // mode), the common cells, then the deferred ones
-    const bool learned = p.precision == HYQ_PREC_MIXED_LEARNED && c->mlp != nullptr;
-    if (learned) {
-      hipLaunchKernelGGL(k_pass1a<true>, dim3(g), dim3(kBlock), 0, c->stream, c->M, c->Mr,
-                         reinterpret_cast<short*>(c->X), c->Xidx, c->Xseg, c->P, c->flags, c->sc,
-                         c->N, p.flag2D, p.Ma, hyq_mlp_input_norm(c->mlp));
-      const int rc = hyq_mlp_infer_bf16_segments_async(
-          c->mlp, reinterpret_cast<const short*>(c->X), c->Xidx, c->Xseg, (c->N + 63) / 64,
-          (int32_t)kSegRows, c->P, c->stream);
-      if (rc) return rc;
-    } else {
-      hipLaunchKernelGGL(k_pass1a<false>, dim3(g), dim3(kBlock), 0, c->stream, c->M, c->Mr,
-                         (short*)nullptr, (unsigned*)nullptr, (unsigned*)nullptr, (float*)nullptr,
-                         c->flags, c->sc, c->N, p.flag2D, p.Ma, (const float*)nullptr);
-    }
-    const float* P = learned ? (const float*)c->P : (const float*)nullptr;
-    hipLaunchKernelGGL(k_pass1_fast<float>, dim3(g), dim3(kBlock), 0, c->stream, (const double*)c->Mr,
-                       (float*)c->vp, c->flags, P, c->L, c->sc, c->N, p.positivity);
-    hipLaunchKernelGGL(k_slot_solve<true>, dim3(kListBlocks), dim3(kBlock), 0, c->stream, c->L,
-                       (const unsigned*)&c->sc->nslot1, &c->sc->nitem1, P, c->sc, c->N);
-    hipLaunchKernelGGL(k_pass1_fixup<float>, dim3(kListBlocks), dim3(kBlock), 0, c->stream, c->L,
-                       (float*)c->vp, c->flags, c->sc, c->N);
-    enqueue_full1<float>(c->stream, c->Mr, (float*)c->F, (float*)c->vp, c->flags, P, c->L,
-                         c->sc, c->N, p.flag2D, p.Ma, p.positivity);
+    hipLaunchKernelGGL((k_project<kBlock, Solo>), dim3(g), dim3(kBlock), 0, c->stream, R, c->M, c->Mr,
+                       c->flags, c->N);
   }
+  launch_planes<EM, 1, FT, Solo>(c->stream, R, g64, c->Mr, vp, c->flags,
+                                 learned ? (const float*)c->P : (const float*)nullptr, c->L,
+                                 &c->sc->cnt, c->N);
+  hipLaunchKernelGGL((k_close<kBlock, EM, FT, Solo>), dim3(g), dim3(kBlock), 0, c->stream, R, c->Mr, F,
+                     vp, c->flags, c->N);
   if (ev) hipEventRecord(ev[1], c->stream);
   hipLaunchKernelGGL(k_dt, dim3(1), dim3(1), 0, c->stream, c->sc, p.CFL, hmin, p.dtmax, p.Kn);
   if (ev) hipEventRecord(ev[2], c->stream);
-  if (p.precision == HYQ_PREC_FP64) {
-    hipLaunchKernelGGL(k_update<double>, dim3(update_grid(c->N)), dim3(kUpdBlock), 0, c->stream, c->Mr,
-                       (const double*)c->F, (const double*)c->vp, c->M, c->sc, p.Nx, p.Ny, p.Nz,
-                       c->dx, c->dy, c->dz);
-  } else {
-    hipLaunchKernelGGL(k_update<float>, dim3(update_grid(c->N)), dim3(kUpdBlock), 0, c->stream, c->Mr,
-                       (const float*)c->F, (const float*)c->vp, c->M, c->sc, p.Nx, p.Ny, p.Nz,
-                       c->dx, c->dy, c->dz);
-  }
+  hipLaunchKernelGGL(k_update<FT>, dim3(update_grid(c->N)), dim3(kUpdBlock), 0, c->stream, c->Mr,
+                     (const FT*)F, (const FT*)vp, c->M, c->sc, p.Nx, p.Ny, p.Nz, c->dx, c->dy, c->dz);
   if (ev) hipEventRecord(ev[3], c->stream);
-  if (p.precision == HYQ_PREC_FP64) {
-    hipLaunchKernelGGL((k_pass2<false, 0>), dim3(g), dim3(kBlock), 0, c->stream, c->M, c->sc,
-                       c->N, p.flag2D, p.Ma, p.positivity, p.Kn);
-  } else if (!fast) {
-    hipLaunchKernelGGL((k_pass2<true, 0>), dim3(g), dim3(kBlock), 0, c->stream, c->M, c->sc,
-                       c->N, p.flag2D, p.Ma, p.positivity, p.Kn);
-  } else {
-    hipLaunchKernelGGL(k_pass2_check, dim3(g), dim3(kBlock), 0, c->stream, (const double*)c->M,
-                       c->Mr, c->L, c->sc, c->N, p.flag2D, p.Ma);
-    hipLaunchKernelGGL(k_slot_solve<false>, dim3(kFixupBlocks), dim3(kBlock), 0, c->stream, c->L,
-                       (const unsigned*)&c->sc->nslot2, &c->sc->nitem2, (const float*)nullptr, c->sc,
-                       c->N);
-    hipLaunchKernelGGL(k_pass2_fixup, dim3(kFixupBlocks), dim3(kBlock), 0, c->stream, c->Mr, c->L,
-                       c->sc, c->N);
-    hipLaunchKernelGGL(k_full2_stage<1>, dim3(kListBlocks), dim3(kBlock), 0, c->stream, c->L,
-                       c->sc, c->N, p.flag2D, p.Ma, c->Mr, c->M, p.positivity, p.Kn);
-    hipLaunchKernelGGL(k_full2_stage<2>, dim3(kListBlocks), dim3(kBlock), 0, c->stream, c->L,
-                       c->sc, c->N, p.flag2D, p.Ma, c->Mr, c->M, p.positivity, p.Kn);
-    hipLaunchKernelGGL(k_pass2_relax, dim3(g), dim3(kBlock), 0, c->stream, c->M,
-                       (const double*)c->Mr, c->sc, c->N, p.flag2D, p.Ma, p.positivity, p.Kn);
-  }
+  hipLaunchKernelGGL((k_project<kBlock, Solo>), dim3(g), dim3(kBlock), 0, c->stream, R,
+                     (const double*)c->M, c->Mr, (uint32_t*)nullptr, c->N);
+  launch_planes<EM, 2, FT, Solo>(c->stream, R, g64, c->Mr, (FT*)nullptr, (uint32_t*)nullptr,
+                                 (const float*)nullptr, c->L, &c->sc->cnt, c->N);
+  hipLaunchKernelGGL((k_relax<kBlock, kMixed, Solo>), dim3(g), dim3(kBlock), 0, c->stream, R, c->M,
+                     (const double*)c->Mr, c->N);
   if (ev) hipEventRecord(ev[4], c->stream);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(HYQ_EHIP, "kernel launch", e);
   return HYQ_OK;
 }
+static int enqueue_step(hyq_ctx* c, hipEvent_t* ev) {
+  if (c->p.precision == HYQ_PREC_FP64) return enqueue_step_t<double, 0>(c, ev);
+  if (c->p.precision == HYQ_PREC_MIXED) return enqueue_step_t<float, 0>(c, ev);
+  return enqueue_step_t<float, 1>(c, ev);
+}
+
+extern "C" {
 
 static int load_scalars(hyq_ctx* c, double t, long long nn, double tmax, long long nnmax) {
   DevScalars s;
@@ -1587,8 +918,9 @@ int hyq_deferred_cells(hyq_ctx* c, int64_t* pass1, int64_t* pass2) {
   DevScalars s;
   HIPCHK(hipMemcpyAsync(&s, c->sc, sizeof(s), hipMemcpyDeviceToHost, c->stream), "scalars back");
   HIPCHK(hipStreamSynchronize(c->stream), "sync");
-  if (pass1) *pass1 = (int64_t)s.nhard1 + (int64_t)s.nslot1 - (int64_t)s.ncplx1;
-  if (pass2) *pass2 = (int64_t)s.nhard2 + (int64_t)s.nslot2 - (int64_t)s.ncplx2;
+  const StepCounts& n = s.cnt;
+  if (pass1) *pass1 = (int64_t)n.nhard[0] + (int64_t)n.nslot[0] - (int64_t)n.ncplx[0];
+  if (pass2) *pass2 = (int64_t)n.nhard[1] + (int64_t)n.nslot[1] - (int64_t)n.ncplx[1];
   return HYQ_OK;
 }
 
@@ -1597,8 +929,9 @@ int hyq_fast_path_counts(hyq_ctx* c, int64_t* counts) {
   DevScalars s;
   HIPCHK(hipMemcpyAsync(&s, c->sc, sizeof(s), hipMemcpyDeviceToHost, c->stream), "scalars back");
   HIPCHK(hipStreamSynchronize(c->stream), "sync");
-  const unsigned v[8] = {s.nslot1, s.nitem1, s.ncplx1, s.nhard1 - s.ncplx1,
-                         s.nslot2, s.nitem2, s.ncplx2, s.nhard2 - s.ncplx2};
+  const StepCounts& n = s.cnt;
+  const unsigned v[8] = {n.nslot[0], n.npend[0], n.ncplx[0], n.nhard[0] - n.ncplx[0],
+                         n.nslot[1], n.npend[1], n.ncplx[1], n.nhard[1] - n.ncplx[1]};
   for (int k = 0; k < 8; ++k) counts[k] = (int64_t)v[k];
   return HYQ_OK;
 }
@@ -1646,60 +979,53 @@ static int batch_args(const double* M, int64_t n, int32_t precision, const doubl
   return HYQ_OK;
 }
 
-// The fast batch's scratch for n cells, in one block: the step scalars, then the full-path
-// list, the slots and the plane items of FastLists.
-static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
-static size_t fast_batch_bytes(long long n) {
-  const size_t un = (size_t)n;
-  return align256(sizeof(DevScalars)) + 7 * align256(4 * un) + align256(16 * 8 * un) +
-         2 * align256(35 * 8 * un) + align256(6 * 8 * un);
+}  // extern "C"
+
+// Scratch of a batch of n cells: the flux output, which k_close alone writes, holds the
+// z-path states [35][n], the counters, the entries' lists, and the flags when the caller
+// wants none.  The counters take 64-bit atomics: they sit on a double's boundary, ahead of
+// the 32-bit lists, whose length may be odd.
+struct BatchCounts {
+  StepCounts step;
+  unsigned long long wide[kWideRounds + 1];
+};
+constexpr size_t kCountDoubles = sizeof(BatchCounts) / sizeof(double);
+static_assert(kCountDoubles * sizeof(double) == sizeof(BatchCounts), "whole doubles");
+static_assert(35 * sizeof(double) + sizeof(BatchCounts) + kListBytes + sizeof(uint32_t) <= 105 * sizeof(double),
+              "a batch's scratch fits the fluxes");
+// A kernel rather than a memset, so that the launch sequence can be captured in a graph.
+__global__ void k_batch_begin(BatchCounts* n) {
+  clear_counts(&n->step);
+  for (int r = 0; r <= kWideRounds; ++r) n->wide[r] = 0ull;
 }
-static void fast_batch_carve(char* base, long long n, DevScalars** sc, FastLists* L) {
-  const size_t un = (size_t)n;
-  char* p = base;
-  *sc = reinterpret_cast<DevScalars*>(p); p += align256(sizeof(DevScalars));
-  L->cells = reinterpret_cast<int*>(p); p += align256(4 * un);
-  L->slot_cell = reinterpret_cast<int*>(p); p += align256(4 * un);
-  L->slot_mask = reinterpret_cast<unsigned*>(p); p += align256(4 * un);
-  L->slot_bad = reinterpret_cast<unsigned*>(p); p += align256(4 * un);
-  L->slot_fl = reinterpret_cast<uint32_t*>(p); p += align256(4 * un);
-  L->slot_v = reinterpret_cast<double*>(p); p += align256(16 * 8 * un);
-  L->slot_A = reinterpret_cast<double*>(p); p += align256(35 * 8 * un);
-  L->full_S = reinterpret_cast<double*>(p); p += align256(35 * 8 * un);
-  L->full_v = reinterpret_cast<double*>(p); p += align256(6 * 8 * un);
-  L->full_fl = reinterpret_cast<uint32_t*>(p); p += align256(4 * un);
-  L->full_known = reinterpret_cast<unsigned*>(p);
-}
-// Scalars of a batch: active, everything else zero.  A kernel rather than a memset, so that
-// the launch sequence can be captured in a graph.
-__global__ void k_batch_begin(DevScalars* sc) {
-  sc->t = sc->dt = sc->tmax = 0.0;
-  sc->active = 1.0;
-  sc->vmax_bits = 0ull;
-  sc->nn = sc->nnmax = 0;
-  sc->err = 0ull;
-  sc->nhard1 = sc->nhard2 = sc->nslot1 = sc->nslot2 = 0u;
-  sc->nitem1 = sc->nitem2 = sc->ncplx1 = sc->ncplx2 = 0u;
-}
-// Pass 1 of the fast step on a batch (FP64 outputs) with its scratch at `scr`.
-static void enqueue_fast_batch(const double* M, long long n, double Ma, int flag2D, int positivity,
-                               double* Mr, double* F, double* vp, uint32_t* flags, char* scr) {
-  DevScalars* sc;
-  FastLists L;
-  fast_batch_carve(scr, n, &sc, &L);
+// Batches from this size on take their entries through a launch per phase: with most cells on
+// the list (mixtures), one kernel that does every phase of a cell waits on its slowest lane
+// at 1 wave a SIMD.  524288 mixture cells in FP64: the whole batch 10.2 ms with k_hard, 6.75
+// ms wide (7.45 ms as one kernel per pass).
+constexpr long long kWideCells = 200000;
+static_assert(35 * sizeof(double) + sizeof(BatchCounts) / 1000 + kListBytes + sizeof(uint32_t) + kWideBytes <=
+                  105 * sizeof(double), "a large batch's scratch fits the fluxes");
+// Pass 1 of the step on a batch (FP64 outputs), no allocation.
+template <int EM>
+static void enqueue_batch(const double* M, long long n, double Ma, int flag2D, int positivity,
+                          double* Mr, double* F, double* vp, uint32_t* flags) {
+  const Solo R{nullptr, n, flag2D, positivity, Ma, 0.0};
+  BatchCounts* cnt = reinterpret_cast<BatchCounts*>(F + (size_t)35 * n);
+  const Lists L = carve_lists(F, n, kCountDoubles);
+  uint32_t* fl = L.item + 5 * (size_t)n;
+  const WideLists W{fl + (size_t)n,     fl + 2 * (size_t)n, fl + 3 * (size_t)n,
+                    fl + 4 * (size_t)n, fl + 5 * (size_t)n, cnt->wide};
+  if (flags) fl = flags;
   const unsigned g = grid_for(n);
-  hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(1), 0, 0, sc);
-  hipLaunchKernelGGL(k_pass1a<false>, dim3(g), dim3(kBlock), 0, 0, M, Mr, (short*)nullptr,
-                     (unsigned*)nullptr, (unsigned*)nullptr, (float*)nullptr, flags, sc, n, flag2D,
-                     Ma, (const float*)nullptr);
-  hipLaunchKernelGGL(k_pass1_fast<double>, dim3(g), dim3(kBlock), 0, 0, (const double*)Mr, vp, flags,
-                     (const float*)nullptr, L, sc, n, positivity);
-  hipLaunchKernelGGL(k_slot_solve<true>, dim3(kListBlocks), dim3(kBlock), 0, 0, L,
-                     (const unsigned*)&sc->nslot1, &sc->nitem1, (const float*)nullptr, sc, n);
-  hipLaunchKernelGGL(k_pass1_fixup<double>, dim3(kListBlocks), dim3(kBlock), 0, 0, L, vp, flags, sc, n);
-  enqueue_full1<double>(0, Mr, F, vp, flags, (const float*)nullptr, L, sc, n, flag2D, Ma,
-                        positivity);
+  hipLaunchKernelGGL((k_project<kBlock, Solo>), dim3(g), dim3(kBlock), 0, 0, R, M, Mr, fl, n);
+  hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(1), 0, 0, cnt);
+  launch_planes<EM, 1, double, Solo>(0, R, (unsigned)((n + 63) / 64), Mr, vp, fl, (const float*)nullptr,
+                                     L, &cnt->step, n, n >= kWideCells ? &W : nullptr);
+  hipLaunchKernelGGL((k_close<kBlock, EM, double, Solo>), dim3(g), dim3(kBlock), 0, 0, R, Mr, F, vp,
+                     flags, n);
 }
+
+extern "C" {
 
 int hyq_wavespeed_batch(const double* M, int64_t n, double Ma, int32_t flag2D,
                         int32_t positivity, int32_t precision, double* Mr, double* Fx,
@@ -1707,68 +1033,22 @@ int hyq_wavespeed_batch(const double* M, int64_t n, double Ma, int32_t flag2D,
   const int rc = batch_args(M, n, precision, Mr, Fx, Fy, Fz, vp, flags);
   if (rc) return rc;
   if (n == 0) return HYQ_OK;
-  if (precision == HYQ_PREC_FP64) {
-    hipLaunchKernelGGL((k_pass1<double, 0>), dim3(grid_for(n)), dim3(kBlock), 0, 0, M, Mr, Fx, vp,
-                       flags, (DevScalars*)nullptr, (long long)n, flag2D, Ma, positivity);
-    HIPCHK(hipGetLastError(), "pass1 launch");
-    HIPCHK(hipDeviceSynchronize(), "pass1 sync");
-    return HYQ_OK;
-  }
-  void* scr = nullptr;
-  HIPCHK(hipMalloc(&scr, fast_batch_bytes(n)), "fast batch scratch");
-  enqueue_fast_batch(M, n, Ma, flag2D, positivity, Mr, Fx, vp, flags, static_cast<char*>(scr));
-  hipError_t e = hipGetLastError();
-  const hipError_t e2 = hipDeviceSynchronize();
-  if (e == hipSuccess) e = e2;
-  hipFree(scr);
-  if (e != hipSuccess) return fail(HYQ_EHIP, "fast batch", e);
-  return HYQ_OK;
-}
-
-// ---- the same without allocation ---------------------------------------------------------
-// A fixed device array holds the fast batch's scratch, for callers that cannot allocate
-// (graph capture, serving loops).  Each device holds its own copy until the process ends;
-// every call on a device shares it, so calls that overlap on one device race.
-constexpr long long kNoAllocMaxCells = 1LL << 16;
-static __device__ __align__(256) char scratch[(7 * 4 + 16 * 8 + 2 * 35 * 8 + 6 * 8) * kNoAllocMaxCells + 13 * 256];
-static std::mutex g_scratch_mu;
-static void* g_scratch_ptr[256];  // per device: the array's device address, once looked up
-
-static int scratch_address(char** out) {
-  int dev = -1;
-  HIPCHK(hipGetDevice(&dev), "hipGetDevice");
-  if (dev < 0 || dev >= 256) return fail(HYQ_ENODEV, "device index out of range");
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if (!g_scratch_ptr[dev]) {
-    void* p = nullptr;
-    HIPCHK(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)), "hipGetSymbolAddress(scratch)");
-    g_scratch_ptr[dev] = p;
-  }
-  *out = static_cast<char*>(g_scratch_ptr[dev]);
-  return HYQ_OK;
-}
-
-int hyq_wavespeed_batch_noalloc(const double* M, int64_t n, double Ma, int32_t flag2D,
-                                int32_t positivity, int32_t precision, double* Mr, double* Fx,
-                                double* Fy, double* Fz, double* vp, uint32_t* flags) {
-  int rc = batch_args(M, n, precision, Mr, Fx, Fy, Fz, vp, flags);
-  if (rc) return rc;
-  if (n > kNoAllocMaxCells)
-    return fail(HYQ_EINVAL, "hyq_wavespeed_batch_noalloc: at most 65536 cells per call");
-  if (n == 0) return HYQ_OK;
-  if (precision == HYQ_PREC_FP64) {  // no scratch on this path
-    hipLaunchKernelGGL((k_pass1<double, 0>), dim3(grid_for(n)), dim3(kBlock), 0, 0, M, Mr, Fx, vp,
-                       flags, (DevScalars*)nullptr, (long long)n, flag2D, Ma, positivity);
-  } else {
-    if (fast_batch_bytes(n) > sizeof(scratch)) return fail(HYQ_EINVAL, "scratch too small");
-    char* base = nullptr;
-    rc = scratch_address(&base);
-    if (rc) return rc;
-    enqueue_fast_batch(M, n, Ma, flag2D, positivity, Mr, Fx, vp, flags, base);
-  }
+  if (precision == HYQ_PREC_FP64) enqueue_batch<0>(M, n, Ma, flag2D, positivity, Mr, Fx, vp, flags);
+  else enqueue_batch<1>(M, n, Ma, flag2D, positivity, Mr, Fx, vp, flags);
   HIPCHK(hipGetLastError(), "batch launch");
   HIPCHK(hipDeviceSynchronize(), "batch sync");
   return HYQ_OK;
+}
+
+constexpr long long kNoAllocMaxCells = 1LL << 16;
+int hyq_wavespeed_batch_noalloc(const double* M, int64_t n, double Ma, int32_t flag2D,
+                                int32_t positivity, int32_t precision, double* Mr, double* Fx,
+                                double* Fy, double* Fz, double* vp, uint32_t* flags) {
+  const int rc = batch_args(M, n, precision, Mr, Fx, Fy, Fz, vp, flags);
+  if (rc) return rc;
+  if (n > kNoAllocMaxCells)
+    return fail(HYQ_EINVAL, "hyq_wavespeed_batch_noalloc: at most 65536 cells per call");
+  return hyq_wavespeed_batch(M, n, Ma, flag2D, positivity, precision, Mr, Fx, Fy, Fz, vp, flags);
 }
 
 int hyq_eig6_batch(const double* m15, int64_t n, double* wr, double* wi) {

@@ -14,8 +14,10 @@
 #if defined(__HIPCC__)
 #include <hip/hip_runtime.h>
 #define HD __host__ __device__ __forceinline__
+#define HYQ_COLD __host__ __device__ __attribute__((noinline)) static
 #else  // host build of the cell numerics (CPU test harness only)
 #define HD inline
+#define HYQ_COLD static
 #endif
 // Keeps the instruction scheduler from moving instructions across this point (device code;
 // nothing on the host): loads placed before it are all issued before any use after it.
@@ -42,6 +44,12 @@
 
 namespace hyq {
 
+// Element of a plane at a byte offset (32 bits: a plane holds less than 2^29 cells).
+template <typename T>
+HD T at_byte(const T* plane, unsigned off) {
+  return *(const T*)((const char*)plane + off);
+}
+
 constexpr double EPS = 2.220446049250313e-16;
 
 HD constexpr int tpos(int i, int j, int k) {
@@ -65,6 +73,38 @@ HD double pw(double x) {
 HD double jmax(double a, double b) { return (a != a || b != b) ? (a + b) : (a > b ? a : b); }
 HD double jmin(double a, double b) { return (a != a || b != b) ? (a + b) : (a < b ? a : b); }
 HD double jsign(double x) { return x > 0 ? 1.0 : (x < 0 ? -1.0 : x); }
+
+// Quotients by one denominator b.  The device's IEEE division scales both operands, takes the
+// hardware reciprocal through two Newton steps, and corrects the quotient once, 11
+// instructions (one of them at a quarter of the rate) for each quotient.  Here the
+// reciprocal is made once, without the scaling, and each quotient is the product, its
+// residual's correction and the fix-up of zeros, infinities and NaN: 4 instructions.  The
+// same correctly rounded quotient as long as b, 1/b, a/b and the residual (2^-53 of a) are
+// normal numbers.  Host: plain division.
+struct Recip {
+  double b;
+#if defined(__HIP_DEVICE_COMPILE__)
+  double y;
+  HD explicit Recip(double d) : b(d) {
+    y = __builtin_amdgcn_rcp(d);
+    y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+    y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+  }
+  // from an approximation y0 of 1/d, good to about 2^-48: one Newton step
+  HD Recip(double d, double y0) : b(d) { y = __builtin_fma(__builtin_fma(-d, y0, 1.0), y0, y0); }
+  HD double approx() const { return y; }
+  HD double of(double a) const {
+    const double q = a * y;
+    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), y, q), b, a);
+  }
+#else
+  HD explicit Recip(double d) : b(d) {}
+  HD Recip(double d, double) : b(d) {}
+  HD double approx() const { return 0.0; }
+  HD double of(double a) const { return a / b; }
+#endif
+};
+HD double div3(double a) { return Recip(3.0, 1.0 / 3.0).of(a); }
 
 // Host/device constexpr copy for compile-time unrolled loops.
 struct E35T {

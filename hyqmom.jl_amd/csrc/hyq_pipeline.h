@@ -293,12 +293,12 @@ HD void pass1_cell(const double* M, int flag2D, double Ma, bool positivity, doub
 // Maxwellian with the same density, velocity and trace temperature.
 template <bool MIXED = false>
 HD void collision_cell(const double* M, double dt, double Kn, bool positivity, double* Mo) {
-  const double rho = M[0], r = 1.0 / rho;
-  const double um = M[1] / rho, vm = M[5] / rho, wm = M[15] / rho;
-  const double C200 = M[2] / rho - um * um, C020 = M[9] / rho - vm * vm,
-               C002 = M[19] / rho - wm * wm;
-  (void)r;
-  double Th = (C200 + C020 + C002) / 3;
+  const double rho = M[0];
+  const Recip r(rho);
+  const double um = r.of(M[1]), vm = r.of(M[5]), wm = r.of(M[15]);
+  const double C200 = r.of(M[2]) - um * um, C020 = r.of(M[9]) - vm * vm,
+               C002 = r.of(M[19]) - wm * wm;
+  double Th = div3(C200 + C020 + C002);
   if (positivity) Th = jmax(Th, 1e-14);
   const double tc = Kn / (rho * sqrt(Th) * 2);
   double g[35];

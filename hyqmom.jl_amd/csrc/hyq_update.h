@@ -131,10 +131,6 @@ HD UpdOff upd_off(const UpdDir<T>& d, unsigned c) {
   r.f2 = (c + (unsigned)d.o2) * (unsigned)sizeof(FT);
   return r;
 }
-template <typename T>
-HD T at_byte(const T* plane, unsigned off) {
-  return *(const T*)((const char*)plane + off);
-}
 
 // One moment's values along one direction: state and flux at cells j-1, j, j+1.
 template <typename FT>

@@ -173,18 +173,16 @@ int hyq_moments5_batch(const double* M, int64_t n, double* M5, double* C5, doubl
  * consecutive [35][n] blocks.  precision HYQ_PREC_FP64: QR eigen solves;
  * HYQ_PREC_MIXED_NEWTON: the fast step's pass-1 kernels (Sturm test, 2x2 block test of a
  * nearly double pair, Laguerre extremes, QR where those do not decide, full path for the
- * eigenvalue corrections), with scratch the call allocates; needs flags.  Both give FP64
- * outputs. */
+ * eigenvalue corrections); needs flags.  Both give FP64 outputs, and use the flux outputs as
+ * scratch before the fluxes are written. */
 int hyq_wavespeed_batch(const double* M, int64_t n, double Ma, int32_t flag2D,
                         int32_t positivity, int32_t precision, double* Mr, double* Fx,
                         double* Fy, double* Fz, double* vp, uint32_t* flags);
 
-/* hyq_wavespeed_batch without any allocation.  No counterpart in the reference: it is for
- * callers that cannot allocate device memory (code under HIP graph capture, serving loops,
- * harnesses that forbid hipMalloc).  The fast mode's scratch lives in a fixed device array
- * that every GPU holds until the process ends; at most 65536 cells per call (HYQ_EINVAL
- * beyond), and calls that overlap on one GPU race.  Same arguments and results as
- * hyq_wavespeed_batch. */
+/* hyq_wavespeed_batch with a limit of 65536 cells per call (HYQ_EINVAL beyond).  No
+ * counterpart in the reference: it is for callers that cannot allocate device memory (serving
+ * loops, harnesses that forbid hipMalloc).  Same arguments and results as
+ * hyq_wavespeed_batch, which allocates nothing either. */
 int hyq_wavespeed_batch_noalloc(const double* M, int64_t n, double Ma, int32_t flag2D,
                                 int32_t positivity, int32_t precision, double* Mr, double* Fx,
                                 double* Fy, double* Fz, double* vp, uint32_t* flags);

@@ -109,3 +109,18 @@ def host_step(M, Kn, Ma, CFL=0.7, dtmax=1e-2, flag2D=0, t=0.0, tmax=1e9):
                      ctypes.c_double(1.0 / Ny), ctypes.c_double(1.0 / Nz), ctypes.c_double(tmax),
                      ctypes.c_double(t), None)
     return soa.reshape(-1, order="C").reshape((35, N)).T.reshape((Nx, Ny, Nz, 35), order="F"), dt
+
+
+def plane_both(M, q):
+    """Plane q from the 15 moments of its set and from all 35: two arrays of 13 values."""
+    M = _f(M); out = np.zeros(26)
+    k = lib().cell_plane_both(_p(M), q, _p(out))
+    return out[:k], out[k:]
+
+
+def plane_decide(M, em, q, fin, wmin=float("nan"), wmax=float("nan")):
+    """Plane q through the planes kernel's decision and through the one-cell solve: two arrays
+    (ok, complex, min, max, flags)."""
+    M = _f(M); out = np.zeros(10)
+    lib().cell_plane_decide(_p(M), em, q, int(fin), ctypes.c_double(wmin), ctypes.c_double(wmax), _p(out))
+    return out[:5], out[5:]

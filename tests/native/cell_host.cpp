@@ -5,6 +5,7 @@
 #include "../../hyqmom.jl_amd/csrc/hyq_pipeline.h"
 #include "../../hyqmom.jl_amd/csrc/hyq_update.h"
 #include "../../hyqmom.jl_amd/csrc/hyq_fasteig.h"
+#include "../../hyqmom.jl_amd/csrc/hyq_planes.h"
 #include <vector>
 #include <cmath>
 
@@ -179,4 +180,62 @@ extern "C" void cell_fast_eigs_J(const double* J36, double sig, int need_vals, d
   const FastEig fe = fast_eigs_std(J36, NAN, NAN, need_vals != 0, sig);
   out[0] = fe.real ? 1 : 0; out[1] = fe.cplx ? 1 : 0; out[2] = fe.lmin; out[3] = fe.lmax;
   out[4] = fe.iters;
+}
+
+// Plane q (slots UV, UW, VU, VW, WU) of a 35-moment state both ways.  out: the 13 fields of the
+// Plane as plane_of_set gives them from the 15 moments of the plane's set, then as cell_plane
+// gives them from all 35.
+extern "C" int cell_plane_both(const double* M, int q, double* out) {
+  double c[35], M000, um, vm, wm, m[15];
+  raw_to_central4(M, c, M000, um, vm, wm);
+  const Plane b = cell_plane(c, um, vm, wm, q);
+  const SetT sets = plane_sets();
+  for (int t = 0; t < 15; ++t) m[t] = M[sets.m[plane_set(q)][t]];
+  const Plane a = plane_of_set(m, plane_swapped(q));
+  const Plane* p[2] = {&a, &b};
+  for (int k = 0; k < 2; ++k) {
+    const double v[12] = {p[k]->a,   p[k]->sig, p[k]->S11, p[k]->S30, p[k]->S21, p[k]->S12,
+                          p[k]->S03, p[k]->S40, p[k]->S31, p[k]->S22, p[k]->S13, p[k]->S04};
+    for (int t = 0; t < 12; ++t) out[13 * k + t] = v[t];
+    out[13 * k + 12] = p[k]->ok ? 1.0 : 0.0;
+  }
+  return 13;
+}
+
+// Plane q of a state through plane_decide<em, true, true> and plane_solve<em, !fin>.  out, for
+// each: ok, complex, the extremes (0 where the decision does not define them), flags.
+extern "C" void cell_plane_decide(const double* M, int em, int q, int fin, double wmin, double wmax,
+                                  double* out) {
+  double c[35], M000, um, vm, wm;
+  raw_to_central4(M, c, M000, um, vm, wm);
+  const Plane p = cell_plane(c, um, vm, wm, q);
+  const float a = (float)wmin, b = (float)wmax;
+  double v0, v1;
+  uint32_t info = em == 0 ? plane_decide<0, true, true>(p, a, b, fin != 0, v0, v1)
+                          : plane_decide<1, true, true>(p, a, b, fin != 0, v0, v1);
+  if (em == 1) {
+    // a plane the first pass leaves open is taken up again with the block test: its
+    // iterations are those of the second solve
+    double w0, w1;
+    const uint32_t first = plane_decide<1, false, true>(p, a, b, fin != 0, w0, w1);
+    if ((first & kPlState) != kPlOpen) {
+      info = first;
+      v0 = w0;
+      v1 = w1;
+    }
+  }
+  uint32_t fl = 0;
+  EigRes r[2];
+  r[0] = plane_result(info, v0, v1, fin != 0);
+  if (em == 0) r[1] = fin ? plane_solve<0, false>(p, a, b, true, fl) : plane_solve<0, true>(p, a, b, true, fl);
+  else r[1] = fin ? plane_solve<1, false>(p, a, b, true, fl) : plane_solve<1, true>(p, a, b, true, fl);
+  const uint32_t f[2] = {plane_flags(0u, info, fin != 0), fl};
+  for (int k = 0; k < 2; ++k) {
+    const bool vals = r[k].ok && (fin || !r[k].cplx);
+    out[5 * k] = r[k].ok;
+    out[5 * k + 1] = r[k].cplx;
+    out[5 * k + 2] = vals ? r[k].vmin : 0.0;
+    out[5 * k + 3] = vals ? r[k].vmax : 0.0;
+    out[5 * k + 4] = (double)f[k];
+  }
 }

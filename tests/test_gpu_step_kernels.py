@@ -1,0 +1,89 @@
+"""The forms of the step's kernels that a size selects, against one another: every cell's result
+is the same bits whatever the batch or grid around it.  (The values themselves are held
+against the oracle by the parity, golden-run and batch tests.)"""
+import numpy as np
+import pytest
+
+from test_gpu_fast_batch import HYQ_PREC_FP64, HYQ_PREC_MIXED_NEWTON, batch, mixed_cells
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def base():
+    """9912 cells: jets (near-Maxwellian) and stress cells (complex planes, z re-projections),
+    and their results in one batch of each precision."""
+    from hyqmom_amd import _lib as L
+    M = mixed_cells()
+    fn = L.lib().hyq_wavespeed_batch
+    return M, {p: batch(fn, M, p) for p in (HYQ_PREC_FP64, HYQ_PREC_MIXED_NEWTON)}
+
+
+# one cell; around a wave; an odd count; around the 1280 blocks from which a wave takes all
+# planes of its cells; around the 200000 cells from which every phase is a launch of its own
+@pytest.mark.parametrize("n", [1, 63, 65, 4099, 81856, 81857, 199999, 200001])
+@pytest.mark.parametrize("precision", [HYQ_PREC_FP64, HYQ_PREC_MIXED_NEWTON])
+def test_a_cell_does_not_depend_on_its_batch(base, n, precision):
+    from hyqmom_amd import _lib as L
+    M, want = base
+    # a stride that is coprime with the count mixes the two kinds of cells in every wave
+    idx = (np.arange(n, dtype=np.int64) * 4099 + 7) % len(M)
+    got = batch(L.lib().hyq_wavespeed_batch, M[idx], precision)
+    for w, g in zip(want[precision], got):
+        assert np.array_equal(w[..., idx], g, equal_nan=True)
+
+
+def test_a_batch_of_hard_cells_only(base):
+    """Every cell on the correction path, and none: lists of full and of zero length."""
+    from hyqmom_amd import _lib as L
+    M, want = base
+    fl = want[HYQ_PREC_FP64][3]
+    hard = np.nonzero(fl & 0xFF0)[0]
+    easy = np.nonzero((fl & 0xFFF) == 0)[0]
+    assert len(hard) > 100 and len(easy) > 100
+    for sel in (hard, easy):
+        idx = np.resize(sel, 5001)
+        for p in (HYQ_PREC_FP64, HYQ_PREC_MIXED_NEWTON):
+            got = batch(L.lib().hyq_wavespeed_batch, M[idx], p)
+            for w, g in zip(want[p], got):
+                assert np.array_equal(w[..., idx], g, equal_nan=True)
+
+
+def test_batch_in_place_and_without_flags(base):
+    """Mr may be M itself, and the FP64 batch runs without the flags output."""
+    from gpu_util import empty_dev, to_dev, to_host
+    from hyqmom_amd import _lib as L
+    M, want = base
+    n = 777
+    Mr, F, vp = to_dev(np.ascontiguousarray(M[:n].T)), empty_dev((105, n)), empty_dev((6, n))
+    p = F.data_ptr()
+    L.check(L.lib().hyq_wavespeed_batch(Mr.data_ptr(), n, 1.5, 0, 1, HYQ_PREC_FP64, Mr.data_ptr(), p,
+                                        p + 35 * n * 8, p + 70 * n * 8, vp.data_ptr(), None), "batch")
+    for w, g in zip(want[HYQ_PREC_FP64], (Mr, F, vp)):
+        assert np.array_equal(w[..., :n], to_host(g), equal_nan=True)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed", "mixed_newton"])
+def test_step_forms_agree(precision):
+    """A state without variation in z is the same in every plane of any depth; the depths lie
+    below and above the grids from which a wave takes all planes of its cells (pass 1 81920;
+    pass 2 131072, FP64 262144).  Zero gradient in z:
+    Mz = M exactly.  dt is fixed by dtmax."""
+    import hyqmom_amd as H
+    from hyqmom_amd.ensemble import jets_params
+    p0 = jets_params((41, 39, 4), 1.5, 0.01, precision)
+    p0["dtmax"] = 1e-4
+    M0 = H.initial_state(p0)[:, :, 2:3, :]
+    out = {}
+    for Nz in (3, 51, 52, 81, 83, 163, 165):  # 1599 cells a plane
+        p = dict(p0, Nz=Nz)
+        s = H.Solver(p)
+        s.set_state(np.asfortranarray(np.repeat(M0, Nz, axis=2)))
+        s.run(10.0, 4)
+        M = s.get_state()
+        s.close()
+        assert np.array_equal(M, np.repeat(M[:, :, :1, :], Nz, axis=2))
+        out[Nz] = M[:, :, 0, :]
+    assert not np.array_equal(out[3], M0[:, :, 0, :])
+    for Nz in out:
+        assert np.array_equal(out[3], out[Nz]), Nz
