@@ -117,7 +117,14 @@ __global__ void k_dt(DevScalars* sc, double CFL, double hmin, double dtmax, doub
 // FT = double: FP64 fluxes and arithmetic; FT = float: the mixed-precision difference form.
 constexpr int kUpdBlock = 256;  // 128: 2-3% slower; 64: 5-9%; 512: 3% (120x120x60)
 HD inline unsigned update_grid(long long n) { return (unsigned)((n + kUpdBlock - 1) / kUpdBlock); }
-template <typename FT>
+// A thread updates 35 moments one after the other, each a round trip to memory.  A grid too
+// small to fill the chip spreads them over kUpdSplit threads instead (blockIdx.y), which
+// repeat the face data: a launch takes 34 -> 9.4 us at 20x20x1, 36 -> 11 us at 37x29x17
+// (mixed).  With more blocks than CUs the repeats cost as much as the waves give: 48.1 us
+// whole, 49.3 us split at 61x53x37 (468 blocks).
+constexpr int kUpdSplit = 7;
+constexpr unsigned kUpdSplitBelow = 256;  // blocks
+template <typename FT, bool SPLIT>
 __global__ __launch_bounds__(kUpdBlock) void k_update(const double* __restrict__ Mr,
                                                    const FT* __restrict__ F,
                                                    const FT* __restrict__ vp,
@@ -132,7 +139,9 @@ __global__ __launch_bounds__(kUpdBlock) void k_update(const double* __restrict__
   const int j = (int)((c / Nx) % Ny);
   const int k = (int)(c / ((long long)Nx * Ny));
   const double dt = sc->dt;
-  update_cell<FT>(Mr, F, vp, Mout, c, i, j, k, Nx, Ny, Nz, N, dt / dx, dt / dy, dt / dz);
+  constexpr int kPer = SPLIT ? 35 / kUpdSplit : 35;
+  const int n0 = SPLIT ? (int)blockIdx.y * kPer : 0;
+  update_cell<FT>(Mr, F, vp, Mout, c, i, j, k, Nx, Ny, Nz, N, dt / dx, dt / dy, dt / dz, n0, n0 + kPer);
 }
 
 // ---- batch kernels ---------------------------------------------------------------------
@@ -704,8 +713,13 @@ static int enqueue_step_t(hyq_ctx* c, hipEvent_t* ev) {
   if (ev) hipEventRecord(ev[1], c->stream);
   hipLaunchKernelGGL(k_dt, dim3(1), dim3(1), 0, c->stream, c->sc, p.CFL, hmin, p.dtmax, p.Kn);
   if (ev) hipEventRecord(ev[2], c->stream);
-  hipLaunchKernelGGL(k_update<FT>, dim3(update_grid(c->N)), dim3(kUpdBlock), 0, c->stream, c->Mr,
-                     (const FT*)F, (const FT*)vp, c->M, c->sc, p.Nx, p.Ny, p.Nz, c->dx, c->dy, c->dz);
+  const unsigned ub = update_grid(c->N);
+  if (ub < kUpdSplitBelow)
+    hipLaunchKernelGGL((k_update<FT, true>), dim3(ub, kUpdSplit), dim3(kUpdBlock), 0, c->stream, c->Mr,
+                       (const FT*)F, (const FT*)vp, c->M, c->sc, p.Nx, p.Ny, p.Nz, c->dx, c->dy, c->dz);
+  else
+    hipLaunchKernelGGL((k_update<FT, false>), dim3(ub), dim3(kUpdBlock), 0, c->stream, c->Mr,
+                       (const FT*)F, (const FT*)vp, c->M, c->sc, p.Nx, p.Ny, p.Nz, c->dx, c->dy, c->dz);
   if (ev) hipEventRecord(ev[3], c->stream);
   hipLaunchKernelGGL((k_project<kBlock, Solo>), dim3(g), dim3(kBlock), 0, c->stream, R,
                      (const double*)c->M, c->Mr, (uint32_t*)nullptr, c->N);

@@ -158,7 +158,7 @@ HD double upd_value(const UpdDir<T>& d, const UpdVals<FT>& v, double dtdx) {
   return d.mode == 2 ? r : v.m1;
 }
 
-// Combined x/y/z update of cell c (i, j, k) for all 35 moments: Mx + My + Mz - 2M
+// Combined x/y/z update of cell c (i, j, k) for moments n0 .. n1 - 1: Mx + My + Mz - 2M
 // (simulation_runner.jl:516-520); when Nz == 1 the z sweep leaves the value unchanged
 // (apply_flux_update_3d.jl:183), as a line of one cell does.  Mr: state planes [35][N]; F:
 // flux planes [105][N] (x, y, z blocks); vp: wave-speed planes [6][N]; out: [35][N]; N is
@@ -170,14 +170,14 @@ HD double upd_value(const UpdDir<T>& d, const UpdVals<FT>& v, double dtdx) {
 template <typename FT>
 HD void update_cell(const double* Mr, const FT* F, const FT* vp, double* out, long long c, int i,
                     int j, int k, int Nx, int Ny, int Nz, long long N, double dtdx, double dtdy,
-                    double dtdz) {
+                    double dtdz, int n0 = 0, int n1 = 35) {
   const int sy = Nx, sz = Nx * Ny;
   const UpdDir<FT> dx = upd_dir(vp + c, vp + N + c, i, Nx, 1);
   const UpdDir<FT> dy = upd_dir(vp + 2 * N + c, vp + 3 * N + c, j, Ny, sy);
   const UpdDir<FT> dz = upd_dir(vp + 4 * N + c, vp + 5 * N + c, k, Nz, sz);
   const unsigned c32 = (unsigned)c;
   const UpdOff ox = upd_off<FT, FT>(dx, c32), oy = upd_off<FT, FT>(dy, c32), oz = upd_off<FT, FT>(dz, c32);
-  for (int n = 0; n < 35; ++n) {
+  for (int n = n0; n < n1; ++n) {
     const double* m = Mr + (size_t)n * N;
     const double m0 = at_byte(m, c32 * 8u);
     const UpdVals<FT> vx = upd_load(ox, m, F + (size_t)n * N);

@@ -66,8 +66,8 @@ def test_batch_in_place_and_without_flags(base):
 @pytest.mark.parametrize("precision", ["fp64", "mixed", "mixed_newton"])
 def test_step_forms_agree(precision):
     """A state without variation in z is the same in every plane of any depth; the depths lie
-    below and above the grids from which a wave takes all planes of its cells (pass 1 81920;
-    pass 2 131072, FP64 262144).  Zero gradient in z:
+    below and above the grids from which a thread updates all moments of a cell (65536 cells)
+    and a wave takes all planes of its cells (pass 1 81920; pass 2 131072, FP64 262144).  Zero gradient in z:
     Mz = M exactly.  dt is fixed by dtmax."""
     import hyqmom_amd as H
     from hyqmom_amd.ensemble import jets_params
@@ -75,7 +75,7 @@ def test_step_forms_agree(precision):
     p0["dtmax"] = 1e-4
     M0 = H.initial_state(p0)[:, :, 2:3, :]
     out = {}
-    for Nz in (3, 51, 52, 81, 83, 163, 165):  # 1599 cells a plane
+    for Nz in (3, 40, 41, 51, 52, 81, 83, 163, 165):  # 1599 cells a plane
         p = dict(p0, Nz=Nz)
         s = H.Solver(p)
         s.set_state(np.asfortranarray(np.repeat(M0, Nz, axis=2)))
