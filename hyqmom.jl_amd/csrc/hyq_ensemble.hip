@@ -19,6 +19,7 @@
 
 #include "../../include/hyqmom.h"
 #include "hyq_ensemble_kernels.h"
+#include "hyq_hostcopy.h"
 
 using namespace hyq;
 using namespace hyq_ens;
@@ -66,6 +67,25 @@ __global__ void ke_dt(RunDev* R, int nr) {
   q.t += dt;
 }
 
+// A run's state between its cells of the ensemble's planes and a contiguous [35][N] array, so
+// that the host copies it in one piece rather than 35.  TO: into the planes; the run's
+// scalars then start over.
+template <bool TO>
+__global__ __launch_bounds__(256) void ke_strips(double* M, double* S, RunDev* q, long long off, long long N,
+                                                 long long P) {
+  const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
+  const int n = blockIdx.y;
+  if (TO && c == 0 && n == 0) {
+    q->t = 0.0;
+    q->nn = 0;
+    q->active = 0.0;
+    q->err = 0ull;
+  }
+  if (c >= N) return;
+  if (TO) M[(size_t)n * P + off + c] = S[(size_t)n * N + c];
+  else S[(size_t)n * N + c] = M[(size_t)n * P + off + c];
+}
+
 int cand_index(int b) {
   for (int i = 0; i < 3; ++i)
     if (kCand[i] == b) return i;
@@ -89,6 +109,7 @@ struct hyq_ensemble {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+  HostCopy* copy = nullptr;  // the states' copies from and to the host
 };
 
 namespace {
@@ -179,6 +200,9 @@ int hyq_ensemble_create(const hyq_params* runs, int32_t nruns, hyq_ensemble** ou
             hipMalloc(&e->vp, fsz * 6 * e->P) == hipSuccess &&
             hipMalloc(&e->flags, sizeof(uint32_t) * e->P) == hipSuccess;
   for (int i = 0; i < 4 && ok; ++i) ok = hipEventCreate(&e->ev[i]) == hipSuccess;
+  long long largest = 0;
+  for (const RunDev& q : e->runs) largest = q.N > largest ? q.N : largest;
+  if (ok) ok = (e->copy = HostCopy::create(sizeof(double) * 35 * largest)) != nullptr;
   // block tables, one per candidate block size
   for (int ci = 0; ci < 3 && ok; ++ci) {
     std::vector<Blk> tab;
@@ -205,6 +229,7 @@ int hyq_ensemble_destroy(hyq_ensemble* e) {
   (void)hipFree(e->R);
   (void)hipFree(e->M);
   (void)hipFree(e->Mr);
+  delete e->copy;
   (void)hipFree(e->Mbak);
   (void)hipFree(e->F);
   (void)hipFree(e->vp);
@@ -221,27 +246,22 @@ int hyq_ensemble_destroy(hyq_ensemble* e) {
 int hyq_ensemble_set_state(hyq_ensemble* e, int32_t r, const double* M) {
   if (!e || !M || r < 0 || r >= e->nr) return efail(HYQ_EINVAL, "bad argument");
   const RunDev& q = e->runs[r];
+  // Mr is free between steps: each step's pass 1 writes it before anything reads it
+  ECHK(e->copy->to_device(e->Mr, M, sizeof(double) * 35 * q.N, e->stream), "state upload");
+  hipLaunchKernelGGL(ke_strips<true>, dim3((unsigned)((q.N + 255) / 256), 35), dim3(256), 0, e->stream,
+                     e->M, e->Mr, e->R + r, q.off, q.N, e->P);
+  ECHK(hipGetLastError(), "state upload");
   ECHK(hipStreamSynchronize(e->stream), "sync");
-  for (int n = 0; n < 35; ++n)
-    ECHK(hipMemcpy(e->M + (size_t)n * e->P + q.off, M + (size_t)n * q.N, sizeof(double) * q.N,
-                   hipMemcpyHostToDevice), "state upload");
-  RunDev h;
-  ECHK(hipMemcpy(&h, e->R + r, sizeof(RunDev), hipMemcpyDeviceToHost), "run scalars");
-  h.t = 0.0;
-  h.nn = 0;
-  h.active = 0.0;
-  h.err = 0ull;
-  ECHK(hipMemcpy(e->R + r, &h, sizeof(RunDev), hipMemcpyHostToDevice), "run scalars");
   return HYQ_OK;
 }
 
 int hyq_ensemble_get_state(hyq_ensemble* e, int32_t r, double* M) {
   if (!e || !M || r < 0 || r >= e->nr) return efail(HYQ_EINVAL, "bad argument");
   const RunDev& q = e->runs[r];
-  ECHK(hipStreamSynchronize(e->stream), "sync");
-  for (int n = 0; n < 35; ++n)
-    ECHK(hipMemcpy(M + (size_t)n * q.N, e->M + (size_t)n * e->P + q.off, sizeof(double) * q.N,
-                   hipMemcpyDeviceToHost), "state download");
+  hipLaunchKernelGGL(ke_strips<false>, dim3((unsigned)((q.N + 255) / 256), 35), dim3(256), 0, e->stream,
+                     e->M, e->Mr, e->R + r, q.off, q.N, e->P);
+  ECHK(hipGetLastError(), "state download");
+  ECHK(e->copy->to_host(M, e->Mr, sizeof(double) * 35 * q.N, e->stream), "state download");
   return HYQ_OK;
 }
 

@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "../../include/hyqmom.h"
+#include "hyq_hostcopy.h"
 #include "hyq_step_kernels.h"
 #include "hyq_update.h"
 
@@ -577,6 +578,7 @@ struct hyq_ctx {
   float* P;        // [5N][2] seeds of each plane: the network's predictions or the Gaussian's
   Lists L;         // the entries of a pass, in F, which is free then
   double* diag;            // [8] results of the diagnostics
+  HostCopy* copy;          // the state's copies from and to the host
 };
 
 extern "C" {
@@ -625,6 +627,7 @@ int hyq_create(const hyq_params* params, hyq_ctx** out) {
          // nothing left to do)
          hipMemset(c->Xseg, 0, sizeof(unsigned) * ((c->N + 63) / 64)) == hipSuccess;
   if (ok) c->L = carve_lists(c->F, c->N);
+  if (ok) ok = (c->copy = HostCopy::create(sizeof(double) * 35 * c->N)) != nullptr;
   if (!ok) {
     hyq_destroy(c);
     return fail(HYQ_ENOMEM, "device allocation failed");
@@ -653,6 +656,7 @@ int hyq_destroy(hyq_ctx* c) {
   hipFree(c->Xidx);
   hipFree(c->Xseg);
   hipFree(c->P);
+  delete c->copy;
   for (int i = 0; i < kNev * kChunk; ++i)
     if (c->ev[i]) hipEventDestroy(c->ev[i]);
   if (c->stream) hipStreamDestroy(c->stream);
@@ -662,17 +666,13 @@ int hyq_destroy(hyq_ctx* c) {
 
 int hyq_set_state(hyq_ctx* c, const double* M) {
   if (!c || !M) return fail(HYQ_EINVAL, "null argument");
-  HIPCHK(hipMemcpyAsync(c->M, M, sizeof(double) * 35 * c->N, hipMemcpyHostToDevice, c->stream),
-         "set_state copy");
-  HIPCHK(hipStreamSynchronize(c->stream), "set_state sync");
+  HIPCHK(c->copy->to_device(c->M, M, sizeof(double) * 35 * c->N, c->stream), "set_state copy");
   return HYQ_OK;
 }
 
 int hyq_get_state(hyq_ctx* c, double* M) {
   if (!c || !M) return fail(HYQ_EINVAL, "null argument");
-  HIPCHK(hipMemcpyAsync(M, c->M, sizeof(double) * 35 * c->N, hipMemcpyDeviceToHost, c->stream),
-         "get_state copy");
-  HIPCHK(hipStreamSynchronize(c->stream), "get_state sync");
+  HIPCHK(c->copy->to_host(M, c->M, sizeof(double) * 35 * c->N, c->stream), "get_state copy");
   return HYQ_OK;
 }
 
@@ -853,9 +853,7 @@ int hyq_snapshot_fields(hyq_ctx* c, double* C, double* S) {
       hipLaunchKernelGGL(k_snapshot_field<1>, dim3(g), dim3(kBlock), 0, c->stream,
                          (const double*)c->M, c->N, c->Mr);
     HIPCHK(hipGetLastError(), "snapshot field launch");
-    HIPCHK(hipMemcpyAsync(dst, c->Mr, sizeof(double) * 35 * c->N, hipMemcpyDeviceToHost, c->stream),
-           "snapshot field copy");
-    HIPCHK(hipStreamSynchronize(c->stream), "snapshot field sync");
+    HIPCHK(c->copy->to_host(dst, c->Mr, sizeof(double) * 35 * c->N, c->stream), "snapshot field copy");
   }
   return HYQ_OK;
 }
