@@ -104,6 +104,25 @@ struct Recip {
   HD double of(double a) const { return a / b; }
 #endif
 };
+
+// sqrt of v > 0: the compiler's own sequence without its scaling of v below 2^-767 and its
+// test for 0 and infinity, so the same bits from about 2^-960 on (below, the last bit may
+// differ; an infinite v gives NaN).  half_inv: 1 / (2 sqrt(v)) to about 2^-50, on the device.
+HD double sqrt_pos(double v, double& half_inv) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double y = __builtin_amdgcn_rsq(v);
+  double s = v * y, h = 0.5 * y;
+  const double r = __builtin_fma(-h, s, 0.5);
+  h = __builtin_fma(h, r, h);
+  s = __builtin_fma(s, r, s);
+  s = __builtin_fma(__builtin_fma(-s, s, v), h, s);
+  half_inv = h;
+  return __builtin_fma(__builtin_fma(-s, s, v), h, s);
+#else
+  half_inv = 0.0;
+  return sqrt(v);
+#endif
+}
 HD double div3(double a) { return Recip(3.0, 1.0 / 3.0).of(a); }
 
 // Host/device constexpr copy for compile-time unrolled loops.
