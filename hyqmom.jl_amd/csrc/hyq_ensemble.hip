@@ -5,8 +5,9 @@
 // owns cells [off_r, off_r + N_r), each in its own Julia order).  Kernels run over blocks
 // of one run each: a block table maps blockIdx -> (run, first cell), so a block reads its
 // run's parameters and step scalars once and a finished run costs one load per block.
-// One step = five launches (begin, pass 1, dt, update, pass 2) captured once into a graph
-// and replayed; the per-run dt reduction is an atomic max into the run's scalars.
+// One step (begin, pass 1, dt, update, pass 2: the single run's kernels, hyq_step_kernels.h, over
+// the block table) is captured once into a graph and replayed; the per-run dt reduction is an
+// atomic max into the run's scalars.
 //
 // The block size of each of the three cell kernels is a tunable: hyq_ensemble_tune times
 // every candidate on the ensemble's own state (saved and restored around the trial steps)
@@ -43,8 +44,9 @@ int efail(int code, const char* what, hipError_t e = hipSuccess) {
 
 constexpr int kCand[3] = {64, 128, 256};  // block-size candidates
 
-__global__ void ke_begin(RunDev* R, int nr) {
+__global__ void ke_begin(RunDev* R, int nr, StepCounts* cnt) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r == 0) clear_counts(cnt);
   if (r >= nr) return;
   RunDev& q = R[r];
   // a run whose z wave-speed solve met a non-finite Jacobian stops there (the reference throws)
@@ -102,6 +104,7 @@ struct hyq_ensemble {
   double *M = nullptr, *Mr = nullptr, *Mbak = nullptr;
   void *F = nullptr, *vp = nullptr;
   uint32_t* flags = nullptr;
+  StepCounts* cnt = nullptr;
   Blk* T[3] = {nullptr, nullptr, nullptr};
   int nblk[3] = {0, 0, 0};
   int blocks[3] = {128, 128, 128};  // pass 1, update, pass 2
@@ -116,7 +119,9 @@ namespace {
 
 void launch_kernel(hyq_ensemble* e, int which, int b, hipStream_t s) {
   const int ci = cand_index(b);
-  const EnsPtrs p{e->M, e->Mr, e->F, e->vp, e->flags, e->R, e->P};
+  const EnsPtrs p{e->M, e->Mr, e->F, e->vp, e->flags, e->R, e->P, carve_lists(e->F, e->P), e->cnt,
+                  e->T[0], (unsigned)e->nblk[0]};
+  static_assert(kCand[0] == 64, "k_planes runs on blocks of 64 cells");
   if (e->prec == HYQ_PREC_FP64) launch_fp64(which, b, (unsigned)e->nblk[ci], e->T[ci], p, s);
   else if (e->prec == HYQ_PREC_MIXED) launch_mixed(which, b, (unsigned)e->nblk[ci], e->T[ci], p, s);
   else launch_newton(which, b, (unsigned)e->nblk[ci], e->T[ci], p, s);
@@ -125,7 +130,7 @@ void launch_kernel(hyq_ensemble* e, int which, int b, hipStream_t s) {
 // One step; with ev != null, events around the three cell kernels (ev[0..3]).
 void enqueue(hyq_ensemble* e, hipStream_t s, hipEvent_t* ev) {
   const unsigned gr = (unsigned)((e->nr + 63) / 64);
-  hipLaunchKernelGGL(ke_begin, dim3(gr), dim3(64), 0, s, e->R, e->nr);
+  hipLaunchKernelGGL(ke_begin, dim3(gr), dim3(64), 0, s, e->R, e->nr, e->cnt);
   if (ev) hipEventRecord(ev[0], s);
   launch_kernel(e, 0, e->blocks[0], s);
   if (ev) hipEventRecord(ev[1], s);
@@ -198,7 +203,8 @@ int hyq_ensemble_create(const hyq_params* runs, int32_t nruns, hyq_ensemble** ou
             hipMalloc(&e->Mr, sizeof(double) * 35 * e->P) == hipSuccess &&
             hipMalloc(&e->F, fsz * 105 * e->P) == hipSuccess &&
             hipMalloc(&e->vp, fsz * 6 * e->P) == hipSuccess &&
-            hipMalloc(&e->flags, sizeof(uint32_t) * e->P) == hipSuccess;
+            hipMalloc(&e->flags, sizeof(uint32_t) * e->P) == hipSuccess &&
+            hipMalloc(&e->cnt, sizeof(StepCounts)) == hipSuccess;
   for (int i = 0; i < 4 && ok; ++i) ok = hipEventCreate(&e->ev[i]) == hipSuccess;
   long long largest = 0;
   for (const RunDev& q : e->runs) largest = q.N > largest ? q.N : largest;
@@ -234,6 +240,7 @@ int hyq_ensemble_destroy(hyq_ensemble* e) {
   (void)hipFree(e->F);
   (void)hipFree(e->vp);
   (void)hipFree(e->flags);
+  (void)hipFree(e->cnt);
   for (int i = 0; i < 3; ++i) (void)hipFree(e->T[i]);
   for (int i = 0; i < 4; ++i)
     if (e->ev[i]) (void)hipEventDestroy(e->ev[i]);

@@ -4,7 +4,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include "hyq_pipeline.h"
+#include <type_traits>
+
+#include "hyq_step_kernels.h"
 #include "hyq_update.h"
 
 namespace hyq_ens {
@@ -24,48 +26,37 @@ struct Blk {
   long long first;
 };
 
-__device__ __forceinline__ unsigned long long ewave_max(unsigned long long v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const unsigned long long w = __shfl_xor(v, o);
-    v = w > v ? w : v;
+// The runs of an ensemble to the step's kernels: a block is one run's (block table T of the
+// kernel's block size).
+struct EnsRun {
+  static constexpr bool kRoundFast = false, kWide = false;
+  RunDev* R;
+  const Blk* T;
+  __device__ __forceinline__ CellCtx of_run(int run) const {
+    RunDev* q = R + run;
+    CellCtx x;
+    x.active = q->active != 0.0;
+    x.in = false;
+    x.c = 0;
+    x.run = run;
+    x.flag2D = q->flag2D;
+    x.positivity = q->positivity;
+    x.Ma = q->Ma;
+    x.Kn = q->Kn;
+    x.dt = q->dt;
+    x.vmax = &q->vmax_bits;
+    x.err = &q->err;
+    return x;
   }
-  return v;
-}
-
-// at least two waves per SIMD: as for the single-run kernels, latency hiding pays for the
-// spills this forces
-template <int B, typename FT, int EM>
-__global__ __launch_bounds__(B, 2) void ke_pass1(const double* __restrict__ M, double* __restrict__ Mr,
-                                              FT* __restrict__ F, FT* __restrict__ vp,
-                                              uint32_t* __restrict__ flags, RunDev* R,
-                                              const Blk* __restrict__ T, long long P) {
-  const Blk b = T[blockIdx.x];
-  RunDev* q = R + b.run;
-  if (q->active == 0.0) return;
-  const long long c = b.first + threadIdx.x;
-  unsigned long long vb = 0;
-  if (c < q->off + q->N) {
-    double m[35], mr[35], v[6];
-#pragma unroll
-    for (int n = 0; n < 35; ++n) m[n] = M[(size_t)n * P + c];
-    uint32_t fl = 0;
-    pass1_cell<FT, EM>(m, q->flag2D, q->Ma, q->positivity != 0, mr, F + c, F + (size_t)35 * P + c,
-                       F + (size_t)70 * P + c, (size_t)P, v, fl);
-#pragma unroll
-    for (int n = 0; n < 35; ++n) Mr[(size_t)n * P + c] = mr[n];
-#pragma unroll
-    for (int d = 0; d < 6; ++d) {
-      vp[(size_t)d * P + c] = (FT)v[d];
-      const unsigned long long bits = __double_as_longlong(fabs(v[d]));
-      vb = bits > vb ? bits : vb;
-    }
-    flags[c] = fl;
-    if (fl & F_NONFIN) atomicOr(&q->err, 1ull);
+  __device__ __forceinline__ CellCtx entry(const Lists& L, unsigned e) const { return of_run(L.run[e]); }
+  __device__ __forceinline__ CellCtx cell(unsigned block, int, unsigned t) const {
+    const Blk b = T[block];
+    CellCtx x = of_run(b.run);
+    x.c = b.first + t;
+    x.in = x.c < R[b.run].off + R[b.run].N;
+    return x;
   }
-  vb = ewave_max(vb);
-  if ((threadIdx.x & 63) == 0) atomicMax(&q->vmax_bits, vb);
-}
+};
 
 template <int B, typename FT>
 __global__ __launch_bounds__(B) void ke_update(const double* __restrict__ Mr, const FT* __restrict__ F,
@@ -83,52 +74,50 @@ __global__ __launch_bounds__(B) void ke_update(const double* __restrict__ Mr, co
   update_cell<FT>(Mr, F, vp, Mout, c, i, j, k, Nx, Ny, q->Nz, P, dt / q->dx, dt / q->dy, dt / q->dz);
 }
 
-template <int B, bool MIXED, int EM>
-__global__ __launch_bounds__(B, 2) void ke_pass2(double* __restrict__ M, const RunDev* R,
-                                              const Blk* __restrict__ T, long long P) {
-  const Blk b = T[blockIdx.x];
-  const RunDev* q = R + b.run;
-  if (q->active == 0.0) return;
-  const long long c = b.first + threadIdx.x;
-  if (c >= q->off + q->N) return;
-  double m[35], o[35];
-#pragma unroll
-  for (int n = 0; n < 35; ++n) m[n] = M[(size_t)n * P + c];
-  uint32_t fl = 0;
-  pass2_cell<MIXED, EM>(m, q->flag2D, q->Ma, q->positivity != 0, q->dt, q->Kn, o, fl);
-#pragma unroll
-  for (int n = 0; n < 35; ++n) M[(size_t)n * P + c] = o[n];
-}
-
-// Device pointers of the ensemble's planes.
+// Device pointers of the ensemble's planes, its lists (in F) and their counters, and the
+// blocks of 64 cells (which k_planes runs on).
 struct EnsPtrs {
   double *M, *Mr;
   void *F, *vp;
   uint32_t* flags;
   RunDev* R;
   long long P;
+  Lists L;
+  StepCounts* cnt;
+  const Blk* T64;
+  unsigned nblk64;
 };
 
-// Launch one of the three cell kernels (0 pass 1, 1 update, 2 pass 2) with block size b.
+// Launch one of the three phases (0 pass 1, 1 update, 2 pass 2) with block size b for the
+// kernels of every cell.
 template <typename FT, int EM, bool MIXED>
 void launch_cells(int which, int b, unsigned nblk, const Blk* T, const EnsPtrs& p, hipStream_t s) {
   FT* F = (FT*)p.F;
   FT* vp = (FT*)p.vp;
-#define HYQ_EL(B)                                                                                    \
-  do {                                                                                               \
-    if (which == 0)                                                                                  \
-      hipLaunchKernelGGL((ke_pass1<B, FT, EM>), dim3(nblk), dim3(B), 0, s, p.M, p.Mr, F, vp, p.flags, \
-                         p.R, T, p.P);                                                               \
-    else if (which == 1)                                                                             \
-      hipLaunchKernelGGL((ke_update<B, FT>), dim3(nblk), dim3(B), 0, s, p.Mr, F, vp, p.M, p.R, T,     \
-                         p.P);                                                                       \
-    else                                                                                             \
-      hipLaunchKernelGGL((ke_pass2<B, MIXED, EM>), dim3(nblk), dim3(B), 0, s, p.M, p.R, T, p.P);      \
-  } while (0)
-  if (b == 64) HYQ_EL(64);
-  else if (b == 128) HYQ_EL(128);
-  else HYQ_EL(256);
-#undef HYQ_EL
+  const EnsRun R{p.R, T}, R64{p.R, p.T64};
+  auto cells = [&](auto size) {
+    constexpr int B = decltype(size)::value;
+    if (which == 0) {
+      hipLaunchKernelGGL((k_project<B, EnsRun>), dim3(nblk), dim3(B), 0, s, R, (const double*)p.M, p.Mr,
+                         p.flags, p.P);
+      launch_planes<EM, 1, FT, EnsRun>(s, R64, p.nblk64, p.Mr, vp, p.flags, (const float*)nullptr, p.L,
+                                       p.cnt, p.P);
+      hipLaunchKernelGGL((k_close<B, EM, FT, EnsRun>), dim3(nblk), dim3(B), 0, s, R, p.Mr, F, vp, p.flags,
+                         p.P);
+    } else if (which == 1) {
+      hipLaunchKernelGGL((ke_update<B, FT>), dim3(nblk), dim3(B), 0, s, p.Mr, F, vp, p.M, p.R, T, p.P);
+    } else {
+      hipLaunchKernelGGL((k_project<B, EnsRun>), dim3(nblk), dim3(B), 0, s, R, (const double*)p.M, p.Mr,
+                         (uint32_t*)nullptr, p.P);
+      launch_planes<EM, 2, FT, EnsRun>(s, R64, p.nblk64, p.Mr, (FT*)nullptr, (uint32_t*)nullptr,
+                                       (const float*)nullptr, p.L, p.cnt, p.P);
+      hipLaunchKernelGGL((k_relax<B, MIXED, EnsRun>), dim3(nblk), dim3(B), 0, s, R, p.M,
+                         (const double*)p.Mr, p.P);
+    }
+  };
+  if (b == 64) cells(std::integral_constant<int, 64>{});
+  else if (b == 128) cells(std::integral_constant<int, 128>{});
+  else cells(std::integral_constant<int, 256>{});
 }
 
 // per-precision entry points (one translation unit each)

@@ -71,12 +71,15 @@ struct DevScalars {  // device-resident step scalars
 
 // The one run of a context, or a batch (sc null: no step scalars).
 struct Solo {
+  static constexpr bool kRoundFast = true, kWide = true;
   DevScalars* sc;
   long long N;
   int flag2D, positivity;
   double Ma, Kn;
-  __device__ __forceinline__ CellCtx cell() const {
+  __device__ __forceinline__ CellCtx entry(const Lists&, unsigned) const { return all(); }
+  __device__ __forceinline__ CellCtx all() const {
     CellCtx x;
+    x.run = -1;
     x.active = sc == nullptr || sc->active != 0.0;
     x.in = false;
     x.c = 0;
@@ -90,7 +93,7 @@ struct Solo {
     return x;
   }
   __device__ __forceinline__ CellCtx cell(unsigned block, int threads, unsigned t) const {
-    CellCtx x = cell();
+    CellCtx x = all();
     x.c = (long long)block * threads + t;
     x.in = x.c < N;
     return x;

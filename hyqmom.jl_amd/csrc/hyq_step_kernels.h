@@ -1,6 +1,6 @@
-// Device code of the step's cell kernels, shared by the single run and the batches
-// (hyq_kernels.hip).  A kernel takes a `Run` that says which cell a thread has and the
-// parameters and step scalars.
+// Device code of the step's cell kernels, shared by the single run, the batches
+// (hyq_kernels.hip) and the ensemble (hyq_ensemble_kernels.h).  A kernel takes a `Run` that says
+// which cell a thread has and the parameters and step scalars of that cell's run.
 //
 // Pass 1 is project -> planes [-> solve] -> hard -> close, pass 2 project -> planes
 // [-> solve] -> hard -> relax; the brackets are the fast modes' (EM = 1).
@@ -43,10 +43,11 @@ struct Lists {
   double* v;       // [10][cap] the planes' extremes, v[2q], v[2q + 1]
   double* S;       // [35][cap] the state before a z re-projection
   int* cell;       // [cap]
+  int* run;        // [cap] ensemble: the entry's run (else unused)
   uint32_t* info;  // [5][cap] what is known of each plane (plane_decide)
   uint32_t* item;  // [5 cap] open planes: 5 entry + q
 };
-constexpr size_t kListBytes = 10 * 8 + (1 + 5 + 5) * 4;  // per cell, without S
+constexpr size_t kListBytes = 10 * 8 + (1 + 1 + 5 + 5) * 4;  // per cell, without S
 static_assert(35 * sizeof(double) + kListBytes <= 105 * sizeof(float), "the lists fit the FP32 fluxes");
 // Lists for cap cells in F: S, then `skip` doubles the caller has other use for, the rest.
 inline Lists carve_lists(void* F, long long cap, size_t skip = 0) {
@@ -54,7 +55,8 @@ inline Lists carve_lists(void* F, long long cap, size_t skip = 0) {
   L.S = static_cast<double*>(F);
   L.v = L.S + 35 * (size_t)cap + skip;
   L.cell = reinterpret_cast<int*>(L.v + 10 * (size_t)cap);
-  L.info = reinterpret_cast<uint32_t*>(L.cell + cap);
+  L.run = L.cell + cap;
+  L.info = reinterpret_cast<uint32_t*>(L.run + cap);
   L.item = L.info + 5 * (size_t)cap;
   return L;
 }
@@ -66,6 +68,7 @@ constexpr int kPlExtraShift = 8;
 struct CellCtx {
   bool active, in;  // active: the same for the whole block
   long long c;
+  int run;  // -1: there is one
   int flag2D, positivity;
   double Ma, Kn, dt;
   unsigned long long *vmax, *err;  // null: not wanted (batches)
@@ -73,11 +76,11 @@ struct CellCtx {
 
 // The wave maximum |vp| in two parts: the 6x6 speeds' where they are found (k_planes, k_hard),
 // in FP64 before they are rounded to FT, and the 1D speeds' in k_close.  The maximum over both
-// kinds is that over the combined speeds.  The fast modes take the maximum of the combined
-// speeds from the rounded 6x6 ones instead, all in k_close.
-template <int EM>
+// kinds is that over the combined speeds.  The single run's fast modes take the maximum of the
+// combined speeds from the rounded 6x6 ones instead (Run::kRoundFast), all in k_close.
+template <int EM, typename Run>
 constexpr bool split_max() {
-  return EM == 0;
+  return EM == 0 || !Run::kRoundFast;
 }
 __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
 #pragma unroll
@@ -183,6 +186,7 @@ __device__ __forceinline__ void sort_out(const CellCtx& x, int lane, bool zs, co
   if (!ent) return;
   const unsigned e = e0 + (unsigned)__popcll(em & below);
   L.cell[e] = (int)x.c;
+  if (x.run >= 0) L.run[e] = x.run;
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     uint32_t f = in[p];
@@ -289,7 +293,7 @@ __global__ __launch_bounds__((kPlaneThreads<SPREAD, PASS>), kPlaneWaves<EM>) voi
     auto at = [&](int t) { return SPREAD ? sm[SPREAD ? t : 0][lane] : at_byte(A + (size_t)t * N, c8); };
     zs = z_special(x.positivity != 0, at(0), at(1), at(2), at(5), at(9), at(15), at(19)) != 0;
   }
-  sort_out<EM, PASS, split_max<EM>(), FT>(x, lane, zs, sv[g], si[g], vp, flags, L, cnt, N);
+  sort_out<EM, PASS, split_max<EM, Run>(), FT>(x, lane, zs, sv[g], si[g], vp, flags, L, cnt, N);
 }
 
 // The 15 moments of plane q (not the same on every lane) of cell c.
@@ -433,7 +437,7 @@ __device__ __forceinline__ bool entry_real(unsigned e, long long c, FT* vp, uint
 // sets kStDone.  ahead: after a correction of x or y, WU is solved along with the planes
 // that are needed in any case (a round less, often for nothing).
 template <int EM, int PASS, typename FT, typename Run>
-__device__ __forceinline__ Work advance(const CellCtx& x, unsigned e, long long c, double* A, FT* vp,
+__device__ __forceinline__ Work advance(const Run& R, unsigned e, long long c, double* A, FT* vp,
                                         uint32_t* flags, const Lists& L, long long N, bool ahead,
                                         uint32_t& st, uint32_t& fl) {
   Work w{0u, 0u, 0u};
@@ -442,9 +446,10 @@ __device__ __forceinline__ Work advance(const CellCtx& x, unsigned e, long long 
   auto speeds = [&](int d, double lo, double hi) {  // direction d's extremes
     vp[(size_t)(2 * d) * N + c] = (FT)lo;
     vp[(size_t)(2 * d + 1) * N + c] = (FT)hi;
-    if (split_max<EM>() && x.vmax != nullptr) {
+    unsigned long long* vmax = split_max<EM, Run>() ? R.entry(L, e).vmax : nullptr;
+    if (vmax != nullptr) {
       const unsigned long long b0 = abs_bits(lo), b1 = abs_bits(hi);
-      raise_max(x.vmax, b0 > b1 ? b0 : b1);
+      raise_max(vmax, b0 > b1 ? b0 : b1);
     }
   };
   while (!(st & kStDone) && !w.op && !w.solve) {
@@ -487,7 +492,7 @@ __device__ __forceinline__ Work advance(const CellCtx& x, unsigned e, long long 
       const int at[7] = {0, 1, 2, 5, 9, 15, 19};
 #pragma unroll
       for (int t = 0; t < 7; ++t) m[t] = A[(size_t)at[t] * N + c];
-      const int z = z_special(x.positivity != 0, m[0], m[1], m[2], m[3], m[4], m[5], m[6]);
+      const int z = z_special(R.entry(L, e).positivity != 0, m[0], m[1], m[2], m[3], m[4], m[5], m[6]);
       if (z) {
         st |= kStSpec;
         for (int t = 0; t < 35; ++t) L.S[(size_t)t * N + e] = A[(size_t)t * N + c];
@@ -589,20 +594,22 @@ __global__ __launch_bounds__(kHardThreads, 1) void k_hard(Run R, double* A, FT* 
   constexpr uint32_t kFin = 1u << 16;  // s_item: 8 owner + plane; s_op: op << 16 | owner
   if (tid < 4) s_stat[tid] = 0u;
   __syncthreads();
+  // An entry's context (R.entry) is read where it is used, not kept: the ensemble's holds
+  // pointers of each lane's run, and kept through the rounds they were spilled under a
+  // branch's execution mask, for some of the lanes only.
   for (unsigned first = blockIdx.x * per; first < n; first += gridDim.x * per) {
     const bool mine = tid < per && first + tid < n;
     const unsigned e = first + tid;
     const long long c = mine ? L.cell[e] : 0;
-    const CellCtx x = R.cell();
     uint32_t fl = PASS == 1 && mine ? flags[c] & 0xFFFFu : 0u;
     uint32_t st = mine ? 0u : kStDone;
     if (EM == 1 && mine &&
-        entry_real<PASS, FT>(e, c, vp, flags, L, N, split_max<EM>() ? x.vmax : nullptr, s_stat))
+        entry_real<PASS, FT>(e, c, vp, flags, L, N, split_max<EM, Run>() ? R.entry(L, e).vmax : nullptr, s_stat))
       st = kStDone;
     if (tid == 0) s_nop = s_nitem = 0u;
     __syncthreads();
     for (;;) {
-      const Work w = advance<EM, PASS, FT, Run>(x, e, c, A, vp, flags, L, N, per < 64u, st, fl);
+      const Work w = advance<EM, PASS, FT, Run>(R, e, c, A, vp, flags, L, N, per < 64u, st, fl);
       if (w.op) {
         s_op[atomicAdd(&s_nop, 1u)] = tid | (w.op << 16);
         s_fl[tid] = 0u;
@@ -618,7 +625,7 @@ __global__ __launch_bounds__(kHardThreads, 1) void k_hard(Run R, double* A, FT* 
       if (nop + nitem == 0u) break;  // the same on every thread
       if (slot < nop) {
         const unsigned o = s_op[slot] & 0xFFFFu, oe = first + o;
-        s_fl[o] = apply_op(R.cell(), s_op[slot] >> 16, oe, L.cell[oe], A, L, N);
+        s_fl[o] = apply_op(R.entry(L, oe), s_op[slot] >> 16, oe, L.cell[oe], A, L, N);
       }
       __syncthreads();
       for (unsigned k = slot; k < nitem; k += kHardThreads) {
@@ -668,11 +675,11 @@ __global__ __launch_bounds__(256) void k_wide_advance(Run R, int round, double* 
     Work w{0u, 0u, 0u};
     if (in) {
       const long long c = L.cell[e];
-      const CellCtx x = R.cell();
       uint32_t st = round == 0 ? 0u : W.st[e], fl = round == 0 ? flags[c] & 0xFFFFu : W.fl[e];
-      if (EM == 1 && round == 0 && entry_real<1, double>(e, c, vp, flags, L, N, x.vmax, nullptr)) st = kStDone;
+      if (EM == 1 && round == 0 && entry_real<1, double>(e, c, vp, flags, L, N, R.entry(L, e).vmax, nullptr))
+        st = kStDone;
       if (!(st & kStDone) || round == 0) {
-        w = advance<EM, 1, double, Run>(x, e, c, A, vp, flags, L, N, false, st, fl);
+        w = advance<EM, 1, double, Run>(R, e, c, A, vp, flags, L, N, false, st, fl);
         W.st[e] = st;
         W.fl[e] = fl;
       }
@@ -711,7 +718,7 @@ __global__ __launch_bounds__(128, 2) void k_wide_close(Run R, int round, double*
   const unsigned n = (unsigned)W.n[round];
   for (unsigned k = blockIdx.x * 128u + threadIdx.x; k < n; k += gridDim.x * 128u) {
     const unsigned e = W.ope[k];
-    W.fl[e] |= apply_op(R.cell(), W.opb[k], e, L.cell[e], A, L, N);
+    W.fl[e] |= apply_op(R.entry(L, e), W.opb[k], e, L.cell[e], A, L, N);
   }
 }
 template <int EM>
@@ -772,7 +779,7 @@ __global__ __launch_bounds__(B, kCloseWaves) void k_close(Run R, double* __restr
 #pragma unroll
     for (int d = 0; d < 6; ++d) {
       vp[(size_t)d * N + c] = (FT)vd[d];
-      const unsigned long long b = abs_bits(split_max<EM>() ? s1[d] : vd[d]);
+      const unsigned long long b = abs_bits(split_max<EM, Run>() ? s1[d] : vd[d]);
       vb = b > vb ? b : vb;
     }
 #pragma unroll
@@ -832,7 +839,7 @@ void launch_planes(hipStream_t s, const Run& R, unsigned blocks64, double* A, FT
                        flags, P, L, cnt, N);
     return;
   }
-  if constexpr (PASS == 1 && sizeof(FT) == 8)
+  if constexpr (PASS == 1 && sizeof(FT) == 8 && Run::kWide)
     for (int r = 0; r <= kWideRounds; ++r) {
       hipLaunchKernelGGL((k_wide_advance<EM, Run>), dim3(1024), dim3(256), 0, s, R, r, A, vp, flags, L, *W,
                          (const StepCounts*)cnt, N);

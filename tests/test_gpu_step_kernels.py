@@ -87,3 +87,30 @@ def test_step_forms_agree(precision):
     assert not np.array_equal(out[3], M0[:, :, 0, :])
     for Nz in out:
         assert np.array_equal(out[3], out[Nz]), Nz
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed", "mixed_newton"])
+def test_a_run_does_not_depend_on_its_ensemble(precision):
+    """93k cells in all, more than the 81920 from which a wave takes all planes of its cells; each
+    run on its own is below.  Odd grids, one of a single plane, and one that has ended."""
+    from hyqmom_amd import initial_state
+    from hyqmom_amd.ensemble import Ensemble, jets_params
+    runs = [jets_params((37, 31, 29), 1.5, 0.01, precision), jets_params((16, 17, 1), 0.7, 0.3, precision),
+            jets_params((41, 33, 33), 0.9, 0.05, precision), jets_params((25, 24, 24), 1.2, 1.0, precision)]
+    runs[3]["tmax"] = 0.004  # ends within the steps
+
+    def run(ps):
+        e = Ensemble(ps)
+        for r, p in enumerate(ps):
+            e.set_state(r, initial_state(p))
+        e.run(5)
+        out = [e.get_state(r) for r in range(len(ps))], e.status()
+        e.close()
+        return out
+
+    M, (t, dt, nn) = run(runs)
+    assert nn[3] < 5
+    for r, p in enumerate(runs):
+        (m,), (t1, dt1, nn1) = run([p])
+        assert np.array_equal(M[r], m, equal_nan=True), r
+        assert (t[r], dt[r], nn[r]) == (t1[0], dt1[0], nn1[0])
