@@ -3,9 +3,13 @@
                               (hipcc, gfx950; each source compiled in its own process, then linked)
   build/libhyqmom_opcount.so  host build of the cell numerics with FLOP counting (g++)
 """
+import glob
 import os
+import re
+import shutil
 import subprocess
 import sys
+import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -38,6 +42,63 @@ def _run(cmd, verbose):
         raise RuntimeError("%s failed" % cmd[0])
 
 
+def masked_copies(asm):
+    """Join blocks of gfx950 assembly whose first vector instructions run before the execution
+    mask is restored: [(function, line, instructions)].  The register allocator has placed
+    spill copies there, so that only the lanes of the branch before the join were saved and
+    the others went on with what the spill slot held."""
+    lines = asm.split("\n")
+    targets = set(re.findall(r"s_cbranch_execz (\.LBB\d+_\d+)", asm))
+    found, fn, last = [], None, ""
+    narrowed = restored = False  # the block began right after the mask was narrowed; it was widened again
+    for i, line in enumerate(lines):
+        m = re.match(r"^([A-Za-z_]\S*):\s", line)
+        if m:
+            fn, narrowed = m[1], False
+        label, fall = re.match(r"^(\.LBB\d+_\d+):", line), re.match(r"^; %bb\.\d+:", line)
+        if label or fall:
+            if (label and label[1] in targets) or (fall and narrowed and not restored):
+                vec = []
+                for t in lines[i + 1:]:
+                    if t.startswith((".LBB", ".Lfunc", "; %bb")):
+                        break
+                    t = t.split(";")[0].strip()
+                    if t.startswith("s_or_b64 exec, exec"):
+                        if vec:
+                            found.append((fn, i + 1, vec))
+                        break
+                    if "exec" in t or re.match(r"s_(cbranch|branch|swappc|endpgm|setpc)", t):
+                        break
+                    if re.match(r"(v_(?!writelane|readlane)|scratch_|global_|flat_|ds_|buffer_)", t):
+                        vec.append(t)
+            narrowed = bool(re.match(r"s_and_saveexec|s_andn?2?_b64 exec", last))
+            restored = False
+        t = line.split(";")[0].strip()
+        if t and not line.startswith((".", ";")):
+            last = t
+            restored = restored or bool(re.match(r"s_(or|mov)_b64 exec", t))
+    return found
+
+
+def _compile(cmd, obj, verbose):
+    """One object, with its assembly checked for masked_copies."""
+    tmp = tempfile.mkdtemp(dir=os.path.dirname(obj))
+    try:
+        part = os.path.join(tmp, os.path.basename(obj))
+        _run(cmd[:cmd.index("-o") + 1] + [part] + cmd[cmd.index("-o") + 2:] + ["-save-temps=obj"], verbose)
+        asm = glob.glob(os.path.join(tmp, "*gfx950*.s"))
+        if not asm:
+            raise RuntimeError("no device assembly of %s" % obj)
+        for f in asm:
+            with open(f) as fh:
+                bad = masked_copies(fh.read())
+            if bad:
+                raise RuntimeError("%s: spill copies under a partial execution mask: %s" % (obj, bad))
+        os.replace(part, obj)
+    finally:
+        shutil.rmtree(tmp, ignore_errors=True)
+
+
 def build(verbose=True):
     out = os.path.join(HERE, "build")
     os.makedirs(out, exist_ok=True)
@@ -45,7 +106,7 @@ def build(verbose=True):
     cmds = [[HIPCC] + FLAGS + extra + ["-c", "-o", o, os.path.join(HERE, "csrc", f)]
             for (f, _, extra), o in zip(SOURCES, objs)]
     with ThreadPoolExecutor(len(cmds)) as ex:
-        list(ex.map(lambda c: _run(c, verbose), cmds))
+        list(ex.map(lambda c, o: _compile(c, o, verbose), cmds, objs))
     target = os.path.join(out, "libhyqmom_hip.so")
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", target + ".tmp"] + objs, verbose)
     os.replace(target + ".tmp", target)
