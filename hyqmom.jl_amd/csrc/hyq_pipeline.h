@@ -89,11 +89,6 @@ HD int plane_fast_status(const Plane& p, float wmin, float wmax, bool need_vals,
   vmax = need_vals ? p.a + p.sig * fe.lmax : 0.0;
   return kPlaneProven;
 }
-HD bool plane_fast(const Plane& p, float wmin, float wmax, bool need_vals, uint32_t& fl,
-                   double& vmin, double& vmax) {
-  return plane_fast_status(p, wmin, wmax, need_vals, fl, vmin, vmax) == kPlaneProven;
-}
-
 // CORRECTS: a complex pair leads to the eigenvalue correction, which replaces the speeds, so
 // a proven complex pair needs no values; after the correction (CORRECTS = false) the
 // reference takes the real parts of whatever the eigenvalues are, so the QR gives them.
@@ -338,14 +333,7 @@ HD void pass2_cell(const double* M, int flag2D, double Ma, bool positivity, doub
   collision_cell<MIXED>(B, dt, Kn, positivity, Mo);
 }
 
-// ---- the fast step with deferred cells (mixed_newton / mixed_learned modes) -----------------
-// Most cells of a step are hyperbolic on every plane with no density clamp or
-// re-projection on the z path: for them pass 1 and pass 2 reduce to closures and the five
-// fast plane solves.  The rest (a QR fallback, a complex-eigenvalue correction, the z
-// path's clamp or re-projection) are deferred to a second kernel that runs the full path
-// on a compacted list, so the rare, register-hungry branches neither widen the common
-// kernel nor hold up its waves.
-
+// ---- parts of the passes, as the step's kernels run them -------------------------------------
 // The five distinct plane Jacobians of a cell, in this order (the z direction's second plane
 // is the y direction's VW, as eigenvalues6z_hyperbolic_3D.jl:117-120 maps it).
 constexpr int kUV = 0, kUW = 1, kVU = 2, kVW = 3, kWU = 4;
@@ -359,53 +347,6 @@ HD Plane cell_plane(const double* c, double um, double vm, double wm, int q) {
   }
 }
 
-// Decisions of a cell's x/y planes kUV, kUW, kVU, kVW, 2 bits per plane q at bit 2q: the
-// plane is hyperbolic, has a complex pair (the eigenvalue correction), or is not decided.
-constexpr unsigned kKnownNone = 0u, kKnownReal = 1u, kKnownComplex = 2u;
-HD unsigned known_of(unsigned known, int q) { return (known >> (2 * q)) & 3u; }
-
-// The fast step's view of a cell's planes in pass 1 (need_vals, five planes) or pass 2 (the
-// x/y checks, four planes).  Returns kPlaneFull when the cell must take the full path
-// (z density clamp or re-projection, eigenvalues6z_hyperbolic_3D.jl:27-104, a complex pair
-// or a non-finite plane); otherwise the planes the fast solve proved have their (vmin, vmax)
-// in v[2q], v[2q + 1], and bit q of `pend` marks each plane that needs its own full solve.
-// Pass 2 (VALS = false) decides all four planes and returns the decisions in `known`; pass 1
-// stops at the first plane that sends the cell to the full path.
-template <bool PAIR = true, bool VALS = true>
-HD int fast_cell_planes(const double* A, bool positivity, const Warm& w, double v[10],
-                        unsigned& pend, uint32_t& fl, unsigned* known = nullptr) {
-  pend = 0;
-  unsigned kn = 0u;
-  if (VALS) {
-    if (positivity && !(A[0] > 0.0)) return kPlaneFull;
-    if (positivity && A[0] > 1e-15) {
-      const double m0 = A[0];
-      const double vx = A[2] / m0 - (A[1] / m0) * (A[1] / m0);
-      const double vy = A[9] / m0 - (A[5] / m0) * (A[5] / m0);
-      const double vz = A[19] / m0 - (A[15] / m0) * (A[15] / m0);
-      if (vx < 0.0 || vy < 0.0 || vz < 0.0) return kPlaneFull;
-    }
-  }
-  double c[35], M000, um, vm, wm;
-  raw_to_central4(A, c, M000, um, vm, wm);
-  const float nan = NAN;
-  bool full = false;
-#pragma unroll
-  for (int q = 0; q < (VALS ? 5 : 4); ++q) {
-    v[2 * q] = v[2 * q + 1] = 0.0;
-    if (VALS && full) continue;
-    const int st = plane_fast_status<PAIR>(cell_plane(c, um, vm, wm, q), VALS ? w.w[2 * q] : nan,
-                                           VALS ? w.w[2 * q + 1] : nan, VALS, fl, v[2 * q],
-                                           v[2 * q + 1]);
-    if (st == kPlaneFull || st == kPlaneComplex) full = true;
-    if (st == kPlaneSolve) pend |= 1u << q;
-    kn |= (st == kPlaneProven ? kKnownReal : (st == kPlaneComplex ? kKnownComplex : kKnownNone)) << (2 * q);
-  }
-  if (known != nullptr) *known = kn;
-  if (full) return kPlaneFull;
-  return pend ? kPlaneSolve : kPlaneProven;
-}
-
 // x/y/z (min, max) from the five planes' extremes, combined as pass 1 of the full path does.
 HD void combine_planes(const double v[10], double v6[6]) {
   v6[0] = jmin(v[2 * kUV], v[2 * kUW]);
@@ -414,17 +355,6 @@ HD void combine_planes(const double v[10], double v6[6]) {
   v6[3] = jmax(v[2 * kVU + 1], v[2 * kVW + 1]);
   v6[4] = jmin(v[2 * kWU], v[2 * kVW]);
   v6[5] = jmax(v[2 * kWU + 1], v[2 * kVW + 1]);
-}
-
-// x/y/z (min, max) of the 6x6 Jacobians of projected state A when the cell takes none of
-// the rare branches.  Returns false when the cell needs the full path or a plane solve.
-HD bool fast_cell_speeds(const double* A, bool positivity, const Warm& w, double v6[6],
-                         uint32_t& fl) {
-  double v[10];
-  unsigned pend;
-  if (fast_cell_planes<true, true>(A, positivity, w, v, pend, fl) != kPlaneProven) return false;
-  combine_planes(v, v6);
-  return true;
 }
 
 // The 1D closure speeds of the x, y and z slices of Mr (simulation_runner.jl:370-372):
@@ -443,83 +373,7 @@ HD void combine_vp(const double s[6], const double v6[6], double vp[6]) {
   }
 }
 
-// The rest of pass 1 for a cell that took none of the rare branches: closure and fluxes of
-// A and the 1D speeds, combined with the 6x6 speeds v6.
-template <typename FT>
-HD void pass1_finish(const double* A, int flag2D, double Ma, double* Mr, FT* Fx, FT* Fy, FT* Fz,
-                     size_t st, const double v6[6], double vp[6], uint32_t& fl) {
-  flux_closure35<true, FT>(A, flag2D, Ma, Mr, Fx, Fy, Fz, st, fl);
-  double s[6];
-  closure1d_all(Mr, s);
-  combine_vp(s, v6, vp);
-}
-
-// Pass 2 of a cell when its x/y planes need no correction: closure, hyperbolicity check of
-// UV, UW, VU, VW, closure, BGK.  Returns false (Mo untouched) when the cell needs the full
-// pass 2.
-// First half: projection of M to A and the hyperbolicity checks of UV, UW, VU, VW.
-// Returns kPlaneProven, kPlaneSolve (bit q of pend: plane q needs its own full solve) or
-// kPlaneFull (the full pass 2).
-template <bool PAIR = true>
-HD int pass2_check_planes(const double* M, int flag2D, double Ma, double* A, unsigned& pend,
-                          uint32_t& fl, unsigned* known = nullptr) {
-  flux_closure35<false, double>(M, flag2D, Ma, A, nullptr, nullptr, nullptr, 0, fl);
-  double v[10];
-  return fast_cell_planes<PAIR, false>(A, false, no_warm(), v, pend, fl, known);
-}
-// The full decision of plane q of projected state A (the fast solve with the pair test, else
-// the QR): kKnownReal, with (v0, v1) its extremes when need_vals; kKnownComplex; or kKnownNone
-// when the plane is not finite.  Either of the last two sends the cell to the full path.
-HD unsigned solve_plane(const double* A, int q, bool need_vals, float wmin, float wmax,
-                        double& v0, double& v1, uint32_t& fl) {
-  double c[35], M000, um, vm, wm;
-  raw_to_central4(A, c, M000, um, vm, wm);
-  const float nan = NAN;
-  const Plane p = cell_plane(c, um, vm, wm, q);
-  const int st = plane_fast_status<true>(p, need_vals ? wmin : nan, need_vals ? wmax : nan,
-                                         need_vals, fl, v0, v1);
-  if (st == kPlaneFull) return kKnownNone;
-  if (st == kPlaneComplex) return kKnownComplex;
-  if (st == kPlaneSolve) {
-    fl |= F_FALLBACK;
-    const EigRes r = plane_eigs(p, fl);
-    if (!r.ok) return kKnownNone;
-    v0 = r.vmin;
-    v1 = r.vmax;
-    return r.cplx ? kKnownComplex : kKnownReal;
-  }
-  return kKnownReal;
-}
-// Pass 2's x or y check of a full-path cell whose two planes (UV, UW or VU, VW) were already
-// decided on this state (known, as fast_cell_planes returns it): the correction of the planes
-// with a complex pair, without solving the planes again, or a copy when there is none; when
-// a decision is missing, eig6_axis.  The same result as eig6_axis with need_vals = false:
-// the decisions came from the same solves on the same state.  Returns true when the state
-// was corrected.
-template <int AXIS>
-HD bool eig6_axis_decided(const double* M, int flag2D, double Ma, double* Mr, uint32_t& fl,
-                          unsigned known) {
-  const unsigned sa = known_of(known, AXIS == 0 ? kUV : kVU);
-  const unsigned sb = known_of(known, AXIS == 0 ? kUW : kVW);
-  if (sa == kKnownNone || sb == kKnownNone) {
-    double d0, d1;
-    return eig6_axis<AXIS, 1>(M, flag2D, Ma, d0, d1, Mr, fl, no_warm(), false);
-  }
-  if (sa == kKnownReal && sb == kKnownReal) {
-#pragma unroll
-    for (int n = 0; n < 35; ++n) Mr[n] = M[n];
-    return false;
-  }
-  double c[35], M000, um, vm, wm;
-  raw_to_central4(M, c, M000, um, vm, wm);
-  axis_correct<AXIS>(c, M000, um, vm, wm, sa == kKnownComplex, sb == kKnownComplex, flag2D, Ma, Mr, fl);
-  return true;
-}
-HD bool pass2_check(const double* M, int flag2D, double Ma, double* A, uint32_t& fl) {
-  unsigned pend;
-  return pass2_check_planes<true>(M, flag2D, Ma, A, pend, fl) == kPlaneProven;
-}
-// Second half: projection of A and BGK.
+// Pass 2 after the x/y corrections: projection of A and BGK.
 template <bool MIXED>
 HD void pass2_relax(const double* A, int flag2D, double Ma, bool positivity, double dt, double Kn,
                     double* Mo, uint32_t& fl) {
@@ -527,13 +381,4 @@ HD void pass2_relax(const double* A, int flag2D, double Ma, bool positivity, dou
   flux_closure35<false, double>(A, flag2D, Ma, B, nullptr, nullptr, nullptr, 0, fl);
   collision_cell<MIXED>(B, dt, Kn, positivity, Mo);
 }
-template <bool MIXED>
-HD bool pass2_fast(const double* M, int flag2D, double Ma, bool positivity, double dt, double Kn,
-                   double* Mo, uint32_t& fl) {
-  double A[35];
-  if (!pass2_check(M, flag2D, Ma, A, fl)) return false;
-  pass2_relax<MIXED>(A, flag2D, Ma, positivity, dt, Kn, Mo, fl);
-  return true;
-}
-
 }  // namespace hyq
