@@ -167,15 +167,33 @@ HD void eig2x2(double a, double b, double c, double d, double& r1, double& i1, d
     i2 = -i1;
   }
 }
+struct House {
+  double v1, v2, beta;
+};
+// The reflector with IEEE divisions, sig = y^2 + z^2 > 0: for a bulge so small that the squares
+// or their quotients leave the normal numbers (states with moments around 1e-40 and below, at
+// the front of a spreading jet, have such bulges).
+HYQ_COLD House house_small(double x, double y, double z, double sig) {
+  const double mu = sqrt(x * x + sig);
+  const double v0 = (x <= 0) ? x - mu : -sig / (x + mu);
+  return {y / v0, z / v0, 2.0 * v0 * v0 / (sig + v0 * v0)};
+}
 // The square root and three divisions of a reflector are half the instructions of a QR step
 // (5 reflectors, 290 multiply-adds on the rows and columns): the reciprocal of sig + v0^2 starts
 // from those of the square root and of v0.  Full divisions and square root -> this form: the
-// QR kernels 5 to 6% faster (120x120x60 FP64 pass 1 1338 -> 1270 us), the same bits.
+// QR kernels QRGAIN, the same bits.
 HD void house(double x, double y, double z, bool three, double& v1, double& v2, double& beta) {
   const double sig = y * y + (three ? z * z : 0.0);
   v1 = y;
   v2 = three ? z : 0.0;
   if (sig == 0.0) { beta = 0.0; return; }
+  if (__builtin_expect(sig < 0x1p-500, 0)) {
+    const House h = house_small(x, y, three ? z : 0.0, sig);
+    v1 = h.v1;
+    v2 = three ? h.v2 : 0.0;
+    beta = h.beta;
+    return;
+  }
   double h;
   const double mu = sqrt_pos(x * x + sig, h);
   const double v0 = (x <= 0) ? x - mu : Recip(x + mu).of(-sig);

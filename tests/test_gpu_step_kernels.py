@@ -63,6 +63,23 @@ def test_batch_in_place_and_without_flags(base):
         assert np.array_equal(w[..., :n], to_host(g), equal_nan=True)
 
 
+@pytest.mark.parametrize("precision", [HYQ_PREC_FP64, HYQ_PREC_MIXED_NEWTON])
+def test_moments_at_the_underflow_scale(precision):
+    """A cell at the front of a spreading jet (120x120x60, step 19): a Maxwellian of rho = 0.1 but
+    for moments of 1e-26 to 1e-86, whose QR bulges have subnormal squares.  Its speeds are the
+    Maxwellian's, +- sqrt(6) from the 1D closure; the deviations are below 1e-24."""
+    from hyqmom_amd import _lib as L
+    cell = np.array([1e-01, -1.57268323e-26, 1e-01, -4.70059143e-26, 3e-01, 1.34347720e-43, 3.29407251e-26,
+                     5.31150428e-43, 9.86852473e-26, 1e-01, -8.22074091e-26, 1e-01, 5.35310728e-43,
+                     1.78791113e-25, 3e-01, 0.0, -3.98547105e-44, -6.44043138e-63, -1.02113400e-43, 1e-01,
+                     -1.62554612e-26, 1e-01, 0.0, -2.26151976e-43, 3e-01, 0.0, -5.35438946e-86, 6.44062650e-63,
+                     0.0, -1.70396464e-43, 0.0, 1.34347720e-43, 3.34254778e-26, 0.0, 1e-01])
+    got = batch(L.lib().hyq_wavespeed_batch, np.stack([cell] * 3), precision)
+    want = np.sqrt(6.0) * np.array([-1.0, 1.0] * 3)[:, None]
+    assert np.abs(got[2] - want).max() < 1e-12
+    assert np.isfinite(got[1]).all()
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed", "mixed_newton"])
 def test_step_forms_agree(precision):
     """A state without variation in z is the same in every plane of any depth; the depths lie
