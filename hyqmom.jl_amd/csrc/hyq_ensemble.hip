@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -113,6 +114,9 @@ struct hyq_ensemble {
   hipGraphExec_t exec = nullptr;
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   HostCopy* copy = nullptr;  // the states' copies from and to the host
+  // Held by every call that writes Mr: a state travels through it between the host's copy and
+  // the gather or scatter of its cells, and each step's pass 1 writes it.
+  std::mutex mu;
 };
 
 namespace {
@@ -252,6 +256,7 @@ int hyq_ensemble_destroy(hyq_ensemble* e) {
 // State of run r (host, Julia layout (Nx,Ny,Nz,35)); resets the run's t and nn to 0.
 int hyq_ensemble_set_state(hyq_ensemble* e, int32_t r, const double* M) {
   if (!e || !M || r < 0 || r >= e->nr) return efail(HYQ_EINVAL, "bad argument");
+  std::lock_guard<std::mutex> lk(e->mu);
   const RunDev& q = e->runs[r];
   // Mr is free between steps: each step's pass 1 writes it before anything reads it
   ECHK(e->copy->to_device(e->Mr, M, sizeof(double) * 35 * q.N, e->stream), "state upload");
@@ -264,6 +269,7 @@ int hyq_ensemble_set_state(hyq_ensemble* e, int32_t r, const double* M) {
 
 int hyq_ensemble_get_state(hyq_ensemble* e, int32_t r, double* M) {
   if (!e || !M || r < 0 || r >= e->nr) return efail(HYQ_EINVAL, "bad argument");
+  std::lock_guard<std::mutex> lk(e->mu);
   const RunDev& q = e->runs[r];
   hipLaunchKernelGGL(ke_strips<false>, dim3((unsigned)((q.N + 255) / 256), 35), dim3(256), 0, e->stream,
                      e->M, e->Mr, e->R + r, q.off, q.N, e->P);
@@ -290,6 +296,7 @@ int hyq_ensemble_status(hyq_ensemble* e, double* t, double* dt, int64_t* nn) {
 // when use_graph != 0, else direct launches.  Synchronizes before returning.
 int hyq_ensemble_run(hyq_ensemble* e, int64_t nsteps, int32_t use_graph) {
   if (!e || nsteps < 0) return efail(HYQ_EINVAL, "bad argument");
+  std::lock_guard<std::mutex> lk(e->mu);
   if (use_graph && !e->exec) {
     const int rc = build_graph(e);
     if (rc) return rc;
@@ -320,6 +327,7 @@ int hyq_ensemble_set_blocks(hyq_ensemble* e, const int32_t* blocks) {
   if (!e || !blocks) return efail(HYQ_EINVAL, "bad argument");
   for (int i = 0; i < 3; ++i)
     if (cand_index(blocks[i]) < 0) return efail(HYQ_EINVAL, "block size must be 64, 128 or 256");
+  std::lock_guard<std::mutex> lk(e->mu);
   for (int i = 0; i < 3; ++i) e->blocks[i] = blocks[i];
   drop_graph(e);
   return HYQ_OK;
@@ -330,6 +338,7 @@ int hyq_ensemble_set_blocks(hyq_ensemble* e, const int32_t* blocks) {
 // keeps its fastest candidate.  ms_out [3][3] (candidate x kernel) may be NULL.
 int hyq_ensemble_tune(hyq_ensemble* e, int32_t trial_steps, int32_t* blocks_out, double* ms_out) {
   if (!e || trial_steps < 1) return efail(HYQ_EINVAL, "bad argument");
+  std::lock_guard<std::mutex> lk(e->mu);
   if (!e->Mbak) ECHK(hipMalloc(&e->Mbak, sizeof(double) * 35 * e->P), "tuner backup");
   std::vector<RunDev> rbak(e->nr);
   ECHK(hipStreamSynchronize(e->stream), "sync");

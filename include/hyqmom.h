@@ -253,7 +253,8 @@ int hyq_plane_dataset(const double* M, int64_t n, float* X, float* L, uint8_t* v
  * Runs with their own grid, Ma, Kn, CFL and tmax (one precision for all: FP64, MIXED or
  * MIXED_NEWTON) share SoA planes and one HIP-graph-captured step; each run keeps its own
  * CFL dt and loop condition t < tmax.  No counterpart in the reference, which runs one
- * simulation per process (simulation_runner.jl:63). */
+ * simulation per process (simulation_runner.jl:63).  Threads may call set_state, get_state,
+ * run, set_blocks and tune of one ensemble at the same time: the calls wait for one another. */
 typedef struct hyq_ensemble hyq_ensemble;
 int hyq_ensemble_create(const hyq_params* runs, int32_t nruns, hyq_ensemble** out);  // at most 2^29 - 1 cells in all
 int hyq_ensemble_destroy(hyq_ensemble* e);
