@@ -223,7 +223,11 @@ int hyq_ensemble_create(const hyq_params* runs, int32_t nruns, hyq_ensemble** ou
          hipMemcpy(e->T[ci], tab.data(), sizeof(Blk) * tab.size(), hipMemcpyHostToDevice) == hipSuccess;
   }
   if (ok) ok = hipMemcpy(e->R, e->runs.data(), sizeof(RunDev) * nruns, hipMemcpyHostToDevice) == hipSuccess;
-  if (ok) ok = hipMemset(e->M, 0, sizeof(double) * 35 * e->P) == hipSuccess;
+  // on the stream of the calls that follow, which does not wait for the null stream: hipMemset
+  // may return before its fill is done, and a state set next must not be cleared by it
+  if (ok)
+    ok = hipMemsetAsync(e->M, 0, sizeof(double) * 35 * e->P, e->stream) == hipSuccess &&
+         hipStreamSynchronize(e->stream) == hipSuccess;
   if (!ok) {
     hyq_ensemble_destroy(e);
     return efail(HYQ_ENOMEM, "ensemble allocation");

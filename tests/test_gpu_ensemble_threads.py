@@ -1,4 +1,4 @@
-"""Several host threads on one ensemble: each sets and reads its own run while the others do the
+"""The first calls of a new ensemble, and several host threads on one: each sets and reads its own run while the others do the
 same (the calls share one staging buffer on the device), and reads a state while steps run."""
 import threading
 
@@ -44,6 +44,19 @@ def test_threads_on_their_own_runs(sizes):
 
     _together([work(r) for r in range(len(sizes))])
     e.close()
+
+
+def test_the_first_calls_of_a_new_ensemble():
+    """A new ensemble's state is zero, and a state set at once stays (the fill at creation is done
+    before either): 61 MB of planes, an upload of one cell."""
+    from hyqmom_amd.ensemble import Ensemble, jets_params
+    one = np.arange(1.0, 36.0).reshape(1, 1, 1, 35)
+    for k in range(4):
+        e = Ensemble([jets_params((1, 1, 1), 1.0, 0.1, "mixed"), jets_params((60, 60, 60), 1.0, 0.1, "mixed")])
+        e.set_state(0, one)
+        assert np.array_equal(e.get_state(0), one)
+        assert not e.get_state(1).any()
+        e.close()
 
 
 def test_a_state_read_while_steps_run():
