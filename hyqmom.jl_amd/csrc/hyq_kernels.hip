@@ -627,8 +627,10 @@ int hyq_create(const hyq_params* params, hyq_ctx** out) {
          hipMalloc(&c->P, sizeof(float) * 2 * 5 * c->N) == hipSuccess &&
          // no rows until a step's projection has listed some: the network's kernel then
          // reads counts of 0 (it runs, as every kernel of the step, also in a step that has
-         // nothing left to do)
-         hipMemset(c->Xseg, 0, sizeof(unsigned) * ((c->N + 63) / 64)) == hipSuccess;
+         // nothing left to do).  On the steps' own stream, which does not wait for the null
+         // stream, where a fill may outlast its call
+         hipMemsetAsync(c->Xseg, 0, sizeof(unsigned) * ((c->N + 63) / 64), c->stream) == hipSuccess &&
+         hipStreamSynchronize(c->stream) == hipSuccess;
   if (ok) c->L = carve_lists(c->F, c->N);
   if (ok) ok = (c->copy = HostCopy::create(sizeof(double) * 35 * c->N)) != nullptr;
   if (!ok) {

@@ -791,6 +791,19 @@ static int wgrad_rows(long npad) {
 static int wgrad_parts(long npad) { return (int)((npad + wgrad_rows(npad) - 1) / wgrad_rows(npad)); }
 static int row_blocks(long npad) { return (int)std::min<long>((npad / 16 + kRowWaves - 1) / kRowWaves, 256); }
 
+// New parameters (null: zeros) and fresh Adam moments, complete on return: on the network's own
+// stream, which training runs on and which does not wait for the null stream.
+static int fresh_blob(Net* m, const float* blob_host) {
+  if (blob_host)
+    MCHK(hipMemcpyAsync(m->blob, blob_host, sizeof(float) * NBLOB, hipMemcpyHostToDevice, m->stream), "mlp blob");
+  else
+    MCHK(hipMemsetAsync(m->blob, 0, sizeof(float) * NBLOB, m->stream), "mlp blob");
+  MCHK(hipMemsetAsync(m->m1, 0, sizeof(float) * NPARAM, m->stream), "adam m");
+  MCHK(hipMemsetAsync(m->m2, 0, sizeof(float) * NPARAM, m->stream), "adam v");
+  MCHK(hipStreamSynchronize(m->stream), "mlp sync");
+  return HYQ_OK;
+}
+
 static int ensure_cap(Net* m, long npad) {
   if (npad <= m->cap) return HYQ_OK;
   (void)hipFree(m->tr);
@@ -834,13 +847,8 @@ int create(const float* blob_host, void** out) {
     delete m;
     return mfail(HYQ_ENOMEM, "mlp allocation");
   }
-  if (blob_host) {
-    MCHK(hipMemcpy(m->blob, blob_host, sizeof(float) * NBLOB, hipMemcpyHostToDevice), "mlp blob");
-  } else {
-    MCHK(hipMemset(m->blob, 0, sizeof(float) * NBLOB), "mlp blob");
-  }
-  MCHK(hipMemset(m->m1, 0, sizeof(float) * NPARAM), "adam m");
-  MCHK(hipMemset(m->m2, 0, sizeof(float) * NPARAM), "adam v");
+  const int rc = fresh_blob(m, blob_host);
+  if (rc) return rc;
   MCHK(hipMalloc(&m->packed, sizeof(short) * PK_N), "mlp packed weights");
   MCHK(hipMalloc(&m->tpack, sizeof(short) * (PK_N + PT_N)), "mlp packed weights");
   m->shape = -1;
@@ -878,12 +886,10 @@ int get_blob(void* h, float* blob_host) {
 int set_blob(void* h, const float* blob_host) {
   Net* m = static_cast<Net*>(h);
   if (!m || !blob_host) return mfail(HYQ_EINVAL, "null argument");
-  MCHK(hipStreamSynchronize(m->stream), "mlp sync");
-  MCHK(hipMemcpy(m->blob, blob_host, sizeof(float) * NBLOB, hipMemcpyHostToDevice), "mlp blob");
+  const int rc = fresh_blob(m, blob_host);
+  if (rc) return rc;
   m->step = 0;
   m->version += 1;
-  MCHK(hipMemset(m->m1, 0, sizeof(float) * NPARAM), "adam m");
-  MCHK(hipMemset(m->m2, 0, sizeof(float) * NPARAM), "adam v");
   return HYQ_OK;
 }
 
