@@ -46,10 +46,18 @@ def masked_copies(asm):
     """Join blocks of gfx950 assembly whose first vector instructions run before the execution
     mask is restored: [(function, line, instructions)].  The register allocator has placed
     spill copies there, so that only the lanes of the branch before the join were saved and
-    the others went on with what the spill slot held."""
+    the others went on with what the spill slot held.  The joins looked at:
+      - the end of an if: the target of s_cbranch_execz, or the block after one that began by
+        narrowing the mask and has no branch over it;
+      - the end of a loop: the block after `s_andn2_b64 exec` (or s_xor, a loop over the
+        distinct values of a register) and s_cbranch_execnz, where no lane is left;
+      - an else: a block that ends the then side with s_or_saveexec.  What the then side's
+        lanes bring along (v_mov) belongs before it, so only spill copies count there."""
+    copy = re.compile(r"(v_accvgpr_|scratch_)")
+    vector = re.compile(r"(v_(?!writelane|readlane)|scratch_|global_|flat_|ds_|buffer_)")
     lines = asm.split("\n")
     targets = set(re.findall(r"s_cbranch_execz (\.LBB\d+_\d+)", asm))
-    found, fn, last = [], None, ""
+    found, fn, last, before = [], None, "", ""
     narrowed = restored = False  # the block began right after the mask was narrowed; it was widened again
     for i, line in enumerate(lines):
         m = re.match(r"^([A-Za-z_]\S*):\s", line)
@@ -57,25 +65,28 @@ def masked_copies(asm):
             fn, narrowed = m[1], False
         label, fall = re.match(r"^(\.LBB\d+_\d+):", line), re.match(r"^; %bb\.\d+:", line)
         if label or fall:
-            if (label and label[1] in targets) or (fall and narrowed and not restored):
+            loop_end = last.startswith("s_cbranch_execnz") and re.match(r"s_(andn2|xor)_b64 exec, exec", before)
+            if (label and label[1] in targets) or (fall and narrowed and not restored) or loop_end:
                 vec = []
                 for t in lines[i + 1:]:
                     if t.startswith((".LBB", ".Lfunc", "; %bb")):
                         break
                     t = t.split(";")[0].strip()
-                    if t.startswith("s_or_b64 exec, exec"):
+                    if re.match(r"s_or_b64 exec, exec|s_mov_b64 exec, (s\[|vcc)|s_or_saveexec", t):
+                        if t.startswith("s_or_saveexec"):
+                            vec = [v for v in vec if copy.match(v)]
                         if vec:
                             found.append((fn, i + 1, vec))
                         break
                     if "exec" in t or re.match(r"s_(cbranch|branch|swappc|endpgm|setpc)", t):
                         break
-                    if re.match(r"(v_(?!writelane|readlane)|scratch_|global_|flat_|ds_|buffer_)", t):
+                    if vector.match(t):
                         vec.append(t)
             narrowed = bool(re.match(r"s_and_saveexec|s_andn?2?_b64 exec", last))
             restored = False
         t = line.split(";")[0].strip()
         if t and not line.startswith((".", ";")):
-            last = t
+            last, before = t, last
             restored = restored or bool(re.match(r"s_(or|mov)_b64 exec", t))
     return found
 
