@@ -473,16 +473,35 @@ HD EigRes plane_eigs(const Plane& p, uint32_t& fl) {
 // Chebyshev recurrence gives a1, a2, b2, b3; the closure sets a3 = (a1+a2)/2 and scales b3
 // by 5/2; the eigenvalues of the 3x3 Jacobi matrix are the roots of the real cubic
 // (l-a1)(l-a2)(l-a3) - b2 (l-a3) - b3 (l-a1).  Returns min/max real parts.
+struct Jacobi3 {
+  double a1, a2, b2, b3;  // b3 not yet scaled
+};
+// The recurrence with IEEE divisions, for a density or a variance so small that the shared
+// reciprocals overflow (below 2^-1024) or the quotients' corrections underflow.
+HYQ_COLD Jacobi3 jacobi3_small(double m0, double m1, double m2, double m3, double m4) {
+  const double a1 = m1 / m0;
+  const double s33 = m2 - a1 * m1, s34 = m3 - a1 * m2, s35 = m4 - a1 * m3;
+  const double a2 = s34 / s33 - a1, b2 = s33 / m0;
+  const double s44 = s35 - a2 * s34 - b2 * m2;
+  return {a1, a2, b2, s44 / s33};
+}
 HD void closure1d_speeds(double m0, double m1, double m2, double m3, double m4, double& vmin,
                          double& vmax) {
   const Recip r0(m0);
-  const double a1 = r0.of(m1);
+  double a1 = r0.of(m1);
   const double s33 = m2 - a1 * m1, s34 = m3 - a1 * m2, s35 = m4 - a1 * m3;
   const Recip r33(s33);
-  const double a2 = r33.of(s34) - a1;
-  const double b2 = r0.of(s33);
+  double a2 = r33.of(s34) - a1;
+  double b2 = r0.of(s33);
   const double s44 = s35 - a2 * s34 - b2 * m2;
   double b3 = r33.of(s44);
+  if (__builtin_expect(fabs(m0) < 0x1p-900 || fabs(s33) < 0x1p-900, 0)) {
+    const Jacobi3 j = jacobi3_small(m0, m1, m2, m3, m4);
+    a1 = j.a1;
+    a2 = j.a2;
+    b2 = j.b2;
+    b3 = j.b3;
+  }
   const double a3 = (a1 + a2) / 2;
   b3 = b3 * 5.0 / 2.0;
   if (!(fabs(a1) < 1e300 && fabs(a2) < 1e300 && fabs(b2) < 1e300 && fabs(b3) < 1e300)) {

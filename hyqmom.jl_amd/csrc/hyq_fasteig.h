@@ -168,7 +168,7 @@ HD int laguerre_extreme(const double c[7], double& x, int kmax, bool simple) {
       dp = dp * x + p;
       p = p * x + c[t];
     }
-    if (p == 0.0) return it;
+    if (fabs(p) < 0x1p-1000) return it;  // zero, or the correction is lost in x (and 1 / p overflows)
     const Recip rp(p);
     const double G = rp.of(dp);
     const double H = G * G - rp.of(d2p);

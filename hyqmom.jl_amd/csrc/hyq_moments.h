@@ -80,7 +80,12 @@ HD double jsign(double x) { return x > 0 ? 1.0 : (x < 0 ? -1.0 : x); }
 // reciprocal is made once, without the scaling, and each quotient is the product, its
 // residual's correction and the fix-up of zeros, infinities and NaN: 4 instructions.  The
 // same correctly rounded quotient as long as b, 1/b, a/b and the residual (2^-53 of a) are
-// normal numbers.  Host: plain division.
+// normal numbers; a subnormal b whose 1/b overflows gives NaN, so that a denominator that can
+// be that small is tested for (house, closure1d_speeds, laguerre_extreme).  The others cannot:
+// products of standard deviations of at least sqrt(eps) (standardize28), differences of
+// numbers of order 1 (realizability), a column's square sum above 1e-280 (hessenberg_n),
+// leading coefficients of normalized polynomials above 1e-12 (sturm_rem).  Host: plain
+// division.
 struct Recip {
   double b;
 #if defined(__HIP_DEVICE_COMPILE__)
