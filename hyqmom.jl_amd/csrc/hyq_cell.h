@@ -91,7 +91,8 @@ HYQ_COLD void edge_branch(S28* sp, double R110, double R101, double R011, uint32
 }
 
 // Flux_closure35_and_realizable_3D (src/numerics/Flux_closure35_and_realizable_3D.jl:33-234),
-// first half: standardization and the realizability projection (:33-176).
+// first half: standardization and the realizability projection (:33-176).  LOOP: realizable_3D's.
+template <bool LOOP = true>
 HD void closure_project(const double* M4, int flag2D, double Ma, ClosureState& q, uint32_t& fl) {
   const double s3max = 4.0 + fabs(Ma) / 2.0, h2min = 1.0e-8;
   double c[35];
@@ -128,7 +129,7 @@ HD void closure_project(const double* M4, int flag2D, double Ma, ClosureState& q
     // the code: two inlined copies no longer fit the instruction cache
     int left = 0;
     for (bool first = true;; first = false) {
-      const int f220 = realizable_3D(s, fl);
+      const int f220 = realizable_3D<LOOP>(s, fl);
       if (first) {
         if (!f220) break;
         fl |= F_220;
@@ -215,11 +216,11 @@ HD void closure_emit(const ClosureState& q, double* Mr, FT* Fx, FT* Fy, FT* Fz, 
   }
 }
 
-template <bool FLUX, typename FT = double>
+template <bool FLUX, typename FT = double, bool LOOP = true>
 HD void flux_closure35(const double* M4, int flag2D, double Ma, double* Mr, FT* Fx, FT* Fy,
                        FT* Fz, size_t st, uint32_t& fl) {
   ClosureState q;
-  closure_project(M4, flag2D, Ma, q, fl);
+  closure_project<LOOP>(M4, flag2D, Ma, q, fl);
   closure_emit<FLUX, FT>(q, Mr, Fx, Fy, Fz, st);
 }
 

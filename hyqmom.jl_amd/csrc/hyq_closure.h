@@ -467,7 +467,14 @@ HD void edge_corner(double R110, double R101, double R011, S28& s, const P10& p1
 }
 
 // ------------------------------------------------------------------------------------
-// realizable_3D (src/realizability/realizable_3D.jl:39-624).  Returns flag220.
+// realizable_3D (src/realizability/realizable_3D.jl:39-624).  Returns flag220.  LOOP: the six 4x4
+// minors from one copy of the cubic solve (the same bits).  Six inlined copies are a third
+// of the projection's code and set its registers: in the step's projection kernel, which the
+// loop lets fit 255 registers, the loop is faster (134 -> 105 us at 120x120x60).  In a kernel
+// of one wave per SIMD that projects and closes (k_closure_batch), the copies are, where many
+// cells' minors are negative: 524288 mixture cells 616 us with the loop, 547 without; jets 171
+// and 166.
+template <bool LOOP = true>
 HD int realizable_3D(S28& s, uint32_t& fl) {
   int flag220 = 0;
   const double diagmin = 1.0e-10, h2min = 1.0e-10, S2min = 1.0e-12;
@@ -686,24 +693,9 @@ HD int realizable_3D(S28& s, uint32_t& fl) {
 
   // 4x4 minors (:455-608)
   delta2star(s, E);
-  // the six permutations in one loop: one copy of the cubic solve (six inlined ones were a
-  // third of the projection's code and set its registers)
   double mn[6], mx[6];
-#if defined(__HIP_DEVICE_COMPILE__)
-#pragma unroll 1
-#endif
-  for (int k = 0; k < 6; ++k) {
-    Lead4 L;
-    double Sxx;
-    switch (k) {
-      case 0: L = lead4<0>(E); Sxx = s.S220; break;
-      case 1: L = lead4<2>(E); Sxx = s.S220; break;
-      case 2: L = lead4<1>(E); Sxx = s.S202; break;
-      case 3: L = lead4<3>(E); Sxx = s.S202; break;
-      case 4: L = lead4<4>(E); Sxx = s.S022; break;
-      default: L = lead4<5>(E); Sxx = s.S022;
-    }
-    double smin = Sxx, smax = Sxx;
+  auto minor4 = [&](const Lead4& L, double Sxx, double& smin, double& smax) {
+    smin = smax = Sxx;
     if (det4(L) < 0) {
       flag220 = 1;
       fl |= F_R4;
@@ -718,12 +710,37 @@ HD int realizable_3D(S28& s, uint32_t& fl) {
         smax = r3 + d22;
       }
     }
-#pragma unroll
-    for (int j = 0; j < 6; ++j)
-      if (j == k) {
-        mn[j] = smin;
-        mx[j] = smax;
+  };
+  if constexpr (LOOP) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll 1
+#endif
+    for (int k = 0; k < 6; ++k) {
+      Lead4 L;
+      double Sxx, smin, smax;
+      switch (k) {
+        case 0: L = lead4<0>(E); Sxx = s.S220; break;
+        case 1: L = lead4<2>(E); Sxx = s.S220; break;
+        case 2: L = lead4<1>(E); Sxx = s.S202; break;
+        case 3: L = lead4<3>(E); Sxx = s.S202; break;
+        case 4: L = lead4<4>(E); Sxx = s.S022; break;
+        default: L = lead4<5>(E); Sxx = s.S022;
       }
+      minor4(L, Sxx, smin, smax);
+#pragma unroll
+      for (int j = 0; j < 6; ++j)
+        if (j == k) {
+          mn[j] = smin;
+          mx[j] = smax;
+        }
+    }
+  } else {
+    minor4(lead4<0>(E), s.S220, mn[0], mx[0]);
+    minor4(lead4<2>(E), s.S220, mn[1], mx[1]);
+    minor4(lead4<1>(E), s.S202, mn[2], mx[2]);
+    minor4(lead4<3>(E), s.S202, mn[3], mx[3]);
+    minor4(lead4<4>(E), s.S022, mn[4], mx[4]);
+    minor4(lead4<5>(E), s.S022, mn[5], mx[5]);
   }
   const double s220mina = mn[0], s220minb = mn[1], s202mina = mn[2], s202minb = mn[3],
                s022mina = mn[4], s022minb = mn[5];

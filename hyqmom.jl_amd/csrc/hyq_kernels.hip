@@ -160,9 +160,9 @@ __global__ __launch_bounds__(kBlock) void k_closure_batch(const double* __restri
   for (int n = 0; n < 35; ++n) m[n] = M[(size_t)n * N + c];
   uint32_t fl = 0;
   if (Fx != nullptr && Fy != nullptr && Fz != nullptr) {
-    flux_closure35<true>(m, flag2D, Ma, mr, Fx + c, Fy + c, Fz + c, (size_t)N, fl);
+    flux_closure35<true, double, false>(m, flag2D, Ma, mr, Fx + c, Fy + c, Fz + c, (size_t)N, fl);
   } else {
-    flux_closure35<false, double>(m, flag2D, Ma, mr, nullptr, nullptr, nullptr, 0, fl);
+    flux_closure35<false, double, false>(m, flag2D, Ma, mr, nullptr, nullptr, nullptr, 0, fl);
   }
   if (Mr)
 #pragma unroll
