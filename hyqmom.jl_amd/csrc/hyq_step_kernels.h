@@ -435,7 +435,8 @@ __device__ __forceinline__ bool entry_real(unsigned e, long long c, FT* vp, uint
 
 // Takes entry e as far as it gets without new solves; returns the work it then waits for, or
 // sets kStDone.  ahead: after a correction of x or y, WU is solved along with the planes
-// that are needed in any case (a round less, often for nothing).
+// that are needed in any case, a round less and often for nothing: for k_hard, whose rounds
+// are latency (20000 mixture cells in the fast mode 1078 -> 895 us, 30000 1113 -> 850).
 template <int EM, int PASS, typename FT, typename Run>
 __device__ __forceinline__ Work advance(const Run& R, unsigned e, long long c, double* A, FT* vp,
                                         uint32_t* flags, const Lists& L, long long N, bool ahead,
@@ -575,18 +576,27 @@ __device__ __forceinline__ void solve_item(unsigned e, int q, bool fin, long lon
 
 // In one launch, for lists that are short or of unknown length (a step's): a block takes up
 // to kHardThreads entries through all their rounds, with the rounds' lists in LDS.  One wave
-// per SIMD: the time of a short list is the latency of one closure and one solve, which is
-// shortest with the whole register file.
+// per SIMD (WAVES = 1): the time of a short list is the latency of one closure and one solve,
+// which is shortest with the whole register file.  With EM 0 a list of more than
+// kHardEntries, which would take several turns of that form, goes to one of two waves per
+// SIMD (496 B of scratch): a step's first pass on mixtures, us for the step, one wave / two,
+// 61x53x37 2627 / 2195, 120x120x60 15750 / 13360; 100000 mixture cells as a batch 2475 /
+// 1965.  The length is known on the device only, so both are launched, each for its range
+// [lo, hi); the idle one costs 3 us.  With EM 1 the second form needs 832 B of scratch and
+// costs 12 us also when idle, 1.5% of a 120x120x60 step that has no such list.
 constexpr int kHardThreads = 256;
 constexpr unsigned kHardBlocks = 256;  // one per CU
-template <int EM, int PASS, typename FT, typename Run>
-__global__ __launch_bounds__(kHardThreads, 1) void k_hard(Run R, double* A, FT* vp, uint32_t* flags,
-                                                          const float* P, Lists L, StepCounts* cnt,
-                                                          long long N) {
+constexpr unsigned kHardEntries = kHardBlocks * kHardThreads;
+template <int EM, int PASS, int WAVES, typename FT, typename Run>
+__global__ __launch_bounds__(kHardThreads, WAVES) void k_hard(Run R, double* A, FT* vp, uint32_t* flags,
+                                                              const float* P, Lists L, StepCounts* cnt,
+                                                              long long N, unsigned lo, unsigned hi) {
   const unsigned n = (unsigned)cnt->nlist[PASS - 1];
+  if (n < lo || n >= hi) return;
   unsigned per = (n + gridDim.x - 1) / gridDim.x;
   per = per < 1 ? 1 : (per > kHardThreads ? kHardThreads : per);
-  __shared__ unsigned s_nop, s_nitem, s_stat[4];
+  // s_item: final solves from the front, the others from the back
+  __shared__ unsigned s_nop, s_nitem, s_nother, s_stat[4];
   __shared__ uint32_t s_op[kHardThreads], s_fl[kHardThreads], s_item[5 * kHardThreads];
   const unsigned tid = threadIdx.x;
   // work k of a round goes to lane k / waves of wave k % waves: short lists use every SIMD
@@ -606,36 +616,58 @@ __global__ __launch_bounds__(kHardThreads, 1) void k_hard(Run R, double* A, FT* 
     if (EM == 1 && mine &&
         entry_real<PASS, FT>(e, c, vp, flags, L, N, split_max<EM, Run>() ? R.entry(L, e).vmax : nullptr, s_stat))
       st = kStDone;
-    if (tid == 0) s_nop = s_nitem = 0u;
+    if (tid == 0) s_nop = s_nitem = s_nother = 0u;
     __syncthreads();
     for (;;) {
-      const Work w = advance<EM, PASS, FT, Run>(R, e, c, A, vp, flags, L, N, per < 64u, st, fl);
+      const Work w = advance<EM, PASS, FT, Run>(R, e, c, A, vp, flags, L, N, true, st, fl);
       if (w.op) {
         s_op[atomicAdd(&s_nop, 1u)] = tid | (w.op << 16);
         s_fl[tid] = 0u;
       }
       if (w.solve) {
-        unsigned at = atomicAdd(&s_nitem, (unsigned)__popc(w.solve));
+        const uint32_t front = EM == 1 ? w.solve & w.last : w.solve, back = w.solve & ~front;
+        unsigned at = front ? atomicAdd(&s_nitem, (unsigned)__popc(front)) : 0u;
+        unsigned bt = back ? 5u * kHardThreads - 1u - atomicAdd(&s_nother, (unsigned)__popc(back)) : 0u;
 #pragma unroll
-        for (int q = 0; q < 5; ++q)
-          if (w.solve & (1u << q)) s_item[at++] = tid * 8u + (unsigned)q + ((w.last & (1u << q)) ? kFin : 0u);
+        for (int q = 0; q < 5; ++q) {
+          const uint32_t it = tid * 8u + (unsigned)q + ((w.last & (1u << q)) ? kFin : 0u);
+          if (front & (1u << q)) s_item[at++] = it;
+          if (back & (1u << q)) s_item[bt--] = it;
+        }
       }
       __syncthreads();
-      const unsigned nop = s_nop, nitem = s_nitem;
-      if (nop + nitem == 0u) break;  // the same on every thread
+      const unsigned nop = s_nop, nitem = s_nitem, nother = s_nother;
+      if (nop + nitem + nother == 0u) break;  // the same on every thread
       if (slot < nop) {
         const unsigned o = s_op[slot] & 0xFFFFu, oe = first + o;
         s_fl[o] = apply_op(R.entry(L, oe), s_op[slot] >> 16, oe, L.cell[oe], A, L, N);
       }
       __syncthreads();
-      for (unsigned k = slot; k < nitem; k += kHardThreads) {
-        const uint32_t it = s_item[k];
+      // Item k: below nitem the front's, from sep on the back's.  EM 1: a final solve mostly
+      // takes the QR and the others mostly do not, and a wave runs the paths of all its
+      // lanes one after the other, so no wave gets both kinds (mixture cells, 30000 as a batch 893 ->
+      // 845 us, 100000 1900 -> 1630; a 120x120x60 step on them 15240 -> 13720).
+      unsigned k = slot, end = nitem + nother, sep = nitem;
+      if (EM == 1 && nitem != 0u && nother != 0u) {
+        if (nitem <= kHardThreads / 2 && nother <= kHardThreads / 2) {  // two waves each
+          k = (tid & 63u) * 2u + ((tid >> 6) & 1u);
+          if (tid < kHardThreads / 2) end = nitem;
+          else k += nitem;
+        } else {  // the back's from the next whole wave on
+          sep = (nitem + 63u) & ~63u;
+          k = tid;
+          end = sep + nother;
+        }
+      }
+      for (; k < end; k += kHardThreads) {
+        if (k >= nitem && k < sep) continue;
+        const uint32_t it = s_item[k < nitem ? k : 5u * kHardThreads - 1u - (k - sep)];
         const unsigned oe = first + ((it & 0xFFFFu) >> 3);
         solve_item<EM, PASS>(oe, (int)(it & 7u), (it & kFin) != 0u, L.cell[oe], A, P, L, N);
       }
       __syncthreads();
       if (w.op) fl |= s_fl[tid];
-      if (tid == 0) s_nop = s_nitem = 0u;
+      if (tid == 0) s_nop = s_nitem = s_nother = 0u;
       __syncthreads();
     }
     __syncthreads();
@@ -835,8 +867,13 @@ void launch_planes(hipStream_t s, const Run& R, unsigned blocks64, double* A, FT
     hipLaunchKernelGGL(k_solve<PASS>, dim3(kSolveBlocks), dim3(128), 0, s, (const double*)A, P, L,
                        (const StepCounts*)cnt, N);
   if (W == nullptr) {
-    hipLaunchKernelGGL((k_hard<EM, PASS, FT, Run>), dim3(kHardBlocks), dim3(kHardThreads), 0, s, R, A, vp,
-                       flags, P, L, cnt, N);
+    const bool both = EM == 0 && N > kHardEntries;
+    hipLaunchKernelGGL((k_hard<EM, PASS, 1, FT, Run>), dim3(kHardBlocks), dim3(kHardThreads), 0, s, R, A,
+                       vp, flags, P, L, cnt, N, 0u, both ? kHardEntries + 1u : ~0u);
+    if constexpr (EM == 0)
+      if (both)
+        hipLaunchKernelGGL((k_hard<EM, PASS, 2, FT, Run>), dim3(2 * kHardBlocks), dim3(kHardThreads), 0, s,
+                           R, A, vp, flags, P, L, cnt, N, kHardEntries + 1u, ~0u);
     return;
   }
   if constexpr (PASS == 1 && sizeof(FT) == 8 && Run::kWide)
