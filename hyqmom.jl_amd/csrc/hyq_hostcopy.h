@@ -4,9 +4,10 @@
 // pages of a fresh result (another 9 ms for a 242 MB state).  Pinned memory moves at 57 GB/s,
 // and eight threads copy between it and pageable memory faster than that, page faults
 // included.  So large copies go through a ring of pinned chunks, filled or emptied by threads
-// beside the transfers.  Pinned and device pointers, and small arrays, are copied by the
-// runtime as they are.  Down, in ms (runtime / ring): 9 MB 0.52 / 0.41, 34 MB 1.9 / 1.0, 242 MB
-// 22.7 / 5.6; up: 9 MB 0.26 / 0.36, 34 MB 1.04 / 0.97, 108 MB 3.7 / 2.6, 242 MB 8.3 / 5.4.
+// beside the transfers.  Pinned and device pointers, small arrays, and an object's first copies
+// below 32 MiB (early) are copied by the runtime as they are.  Down to fresh pages, in ms (runtime
+// / ring, once it is pinned): 9 MB 0.52 / 0.46, 16 MB 0.89 / 0.66, 34 MB 3.3 / 1.15, 68 MB 6.4 /
+// 1.9, 242 MB 22.6 / 5.6; up: 9 MB 0.26 / 0.36, 34 MB 1.04 / 0.97, 108 MB 3.7 / 2.6, 242 MB 8.3 / 5.4.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -21,7 +22,7 @@ namespace hyq {
 
 class HostCopy {
  public:
-  // Below these the threads' start and the first use's pinning cost what they save.
+  // Below these the threads' start costs what the ring saves.
   static constexpr size_t kMin = size_t(8) << 20, kMinUp = size_t(64) << 20;
 
   // An object for copies of up to `bytes`; its events belong to the current device.
@@ -44,7 +45,8 @@ class HostCopy {
 
   // Both return once the copy is complete.
   hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
-    if (!staged(dst, bytes, kMin)) return direct(dst, src, bytes, hipMemcpyDeviceToHost, s);
+    if (!staged(dst, bytes, kMin) || early(bytes))
+      return direct(dst, src, bytes, hipMemcpyDeviceToHost, s);
     std::lock_guard<std::mutex> lk(mu_);
     const size_t chunk = chunk_of(bytes);
     Team t(static_cast<long>((bytes + chunk - 1) / chunk));
@@ -154,6 +156,21 @@ class HostCopy {
     (void)hipGetLastError();
     return true;
   }
+  // Whether an object's copy down comes too early for the ring: pinning it and giving it back
+  // (in part paid by the next allocation) takes 0.5 to 1.7 ms, and a copy saves 0.05 ms at 9 MB,
+  // 0.23 at 16 and 2.1 at 34.  So below 32 MiB the ring is for objects that have copied about
+  // as often as it takes to make up for that: 13 times at 9 MB, 4 at 16, twice at 25.  An
+  // object that copies once (create, a state up, one down, destroy), ring at once / runtime,
+  // ms: 9 MB 1.4 to 2.4 / 1.0, 16 MB 2.4 to 3.5 / 1.6, 34 MB 3.7 to 6.1 / 5.4, 68 MB 5.2 / 9.9.
+  bool early(size_t bytes) {
+    constexpr size_t kAtOnce = size_t(32) << 20;
+    if (bytes >= kAtOnce) return false;
+    const double r = double(kAtOnce) / bytes;
+    const int n = early_.load();
+    if (n >= std::max(1, (int)(r * r + 0.5))) return false;
+    early_.store(n + 1);
+    return true;
+  }
   bool pin() {
     if (pin_) return true;
     if (hipHostMalloc((void**)&pin_, chunk_of(max_) * kSlots, hipHostMallocPortable) == hipSuccess) return true;
@@ -184,6 +201,7 @@ class HostCopy {
   }
 
   std::mutex mu_;
+  std::atomic<int> early_{0};  // copies down that the ring left to the runtime
   char* pin_ = nullptr;
   hipEvent_t ev_[kSlots] = {};
   size_t max_ = 0;  // of a large object: the largest copy, for which the ring is pinned
