@@ -5,7 +5,7 @@
 // and eight threads copy between it and pageable memory faster than that, page faults
 // included.  So large copies go through a ring of pinned chunks, filled or emptied by threads
 // beside the transfers.  Pinned and device pointers, small arrays, and an object's first copies
-// below 32 MiB (early) are copied by the runtime as they are.  Down to fresh pages, in ms (runtime
+// below 64 MiB (early) are copied by the runtime as they are.  Down to fresh pages, in ms (runtime
 // / ring, once it is pinned): 9 MB 0.52 / 0.46, 16 MB 0.89 / 0.66, 34 MB 3.3 / 1.15, 68 MB 6.4 /
 // 1.9, 242 MB 22.6 / 5.6; up: 9 MB 0.26 / 0.36, 34 MB 1.04 / 0.97, 108 MB 3.7 / 2.6, 242 MB 8.3 / 5.4.
 #pragma once
@@ -157,15 +157,16 @@ class HostCopy {
     return true;
   }
   // Whether an object's copy down comes too early for the ring: pinning it and giving it back
-  // (in part paid by the next allocation) takes 0.5 to 1.7 ms, and a copy saves 0.05 ms at 9 MB,
-  // 0.23 at 16 and 2.1 at 34.  So below 32 MiB the ring is for objects that have copied about
-  // as often as it takes to make up for that: 13 times at 9 MB, 4 at 16, twice at 25.  An
-  // object that copies once (create, a state up, one down, destroy), ring at once / runtime,
-  // ms: 9 MB 1.4 to 2.4 / 1.0, 16 MB 2.4 to 3.5 / 1.6, 34 MB 3.7 to 6.1 / 5.4, 68 MB 5.2 / 9.9.
+  // (in part paid by the next allocation) takes 0.3 to 3 ms, by what pages the system has at
+  // hand, and a copy saves 0.05 ms at 9 MB, 0.23 at 16 and 2.1 at 34.  So below 64 MiB the
+  // ring is for objects that have copied about as often as it takes to make up for that: 13
+  // times at 9 MB, 4 at 16, twice at 25, once from 30 MB on.  An object that copies once
+  // (create, a state up, one down, destroy), ring at once / runtime, ms: 9 MB 1.4 to 2.4 /
+  // 1.0, 16 MB 2.4 to 3.5 / 1.6, 34 MB 3.7 to 6.1 / 5.4, 56 MB 8.0 to 8.7 / 8.4, 68 MB 5.2 to
+  // 9.0 / 9.9.
   bool early(size_t bytes) {
-    constexpr size_t kAtOnce = size_t(32) << 20;
-    if (bytes >= kAtOnce) return false;
-    const double r = double(kAtOnce) / bytes;
+    if (bytes >= kMinUp) return false;
+    const double r = double(size_t(32) << 20) / bytes;
     const int n = early_.load();
     if (n >= std::max(1, (int)(r * r + 0.5))) return false;
     early_.store(n + 1);

@@ -1,5 +1,5 @@
 """A state read many times comes back unchanged each time: the first reads of an object go through
-the runtime, later ones (after 13 at 9 MB, 4 at 16, two at 25) through the ring of pinned chunks;
+the runtime, later ones (after 13 at 9 MB, 4 at 16, two at 25, one at 34) through the ring of pinned chunks;
 and from several threads across the change."""
 import threading
 
