@@ -114,6 +114,7 @@ struct hyq_ensemble {
   hipGraphExec_t exec = nullptr;
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   HostCopy* copy = nullptr;  // the states' copies from and to the host
+  bool ended = false;        // every run was past its end at the last step, and none was set since
   // Held by every call that writes Mr: a state travels through it between the host's copy and
   // the gather or scatter of its cells, and each step's pass 1 writes it.
   std::mutex mu;
@@ -261,6 +262,7 @@ int hyq_ensemble_destroy(hyq_ensemble* e) {
 int hyq_ensemble_set_state(hyq_ensemble* e, int32_t r, const double* M) {
   if (!e || !M || r < 0 || r >= e->nr) return efail(HYQ_EINVAL, "bad argument");
   std::lock_guard<std::mutex> lk(e->mu);
+  e->ended = false;
   const RunDev& q = e->runs[r];
   // Mr is free between steps: each step's pass 1 writes it before anything reads it
   ECHK(e->copy->to_device(e->Mr, M, sizeof(double) * 35 * q.N, e->stream), "state upload");
@@ -305,11 +307,12 @@ int hyq_ensemble_run(hyq_ensemble* e, int64_t nsteps, int32_t use_graph) {
     const int rc = build_graph(e);
     if (rc) return rc;
   }
-  // In pieces, twice as many steps each: a step after the end of every run changes nothing,
-  // and its empty launches take 28 us.
+  // A step after the end of every run changes nothing, and its empty launches take 28 us: no
+  // step is queued once a call has seen that end, and a long call runs in pieces of 32, 64,
+  // ... steps and looks for it after each.
   std::vector<RunDev> h(e->nr);
-  int64_t piece = 8, left = nsteps;
-  for (bool more = true; more; piece *= 2) {
+  int64_t left = e->ended ? 0 : nsteps;
+  for (int64_t piece = 32;; piece *= 2) {
     const int64_t todo = left < piece ? left : piece;
     for (int64_t s = 0; s < todo; ++s) {
       if (use_graph) {
@@ -321,9 +324,12 @@ int hyq_ensemble_run(hyq_ensemble* e, int64_t nsteps, int32_t use_graph) {
     ECHK(hipGetLastError(), "ensemble launch");
     ECHK(hipStreamSynchronize(e->stream), "ensemble sync");
     ECHK(hipMemcpy(h.data(), e->R, sizeof(RunDev) * e->nr, hipMemcpyDeviceToHost), "run scalars");
+    if (todo > 0) {
+      e->ended = true;
+      for (const RunDev& q : h) e->ended = e->ended && q.active == 0.0;
+    }
     left -= todo;
-    more = false;
-    for (int r = 0; r < e->nr; ++r) more = more || (left > 0 && h[r].active != 0.0);
+    if (left == 0 || e->ended) break;
   }
   std::string bad;
   for (int r = 0; r < e->nr; ++r)
