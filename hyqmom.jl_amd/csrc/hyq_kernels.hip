@@ -339,9 +339,9 @@ __global__ __launch_bounds__(kBlock) void k_plane_dataset(const double* __restri
     }
   }
 }
-// The learned mode's projection (k_project) with the network's work: a plane whose standardized moments are within kNetTol of a Gaussian's takes the
-// Gaussian's extreme eigenvalues, -sqrt(3), +sqrt(3), as its seeds (written to P directly;
-// NaN for a plane that is not finite); the others are handed to the network as compacted
+// The learned mode's projection (k_project) with the network's work: a plane whose standardized
+// moments are within kNetTol of a Gaussian's takes the Gaussian's extreme eigenvalues,
+// -sqrt(3), +sqrt(3), as its seeds (written to P directly; NaN for a plane that is not finite); the others are handed to the network as compacted
 // rows, normalized with `norm` (16 means, 16 standard deviations) and rounded to bf16 as the
 // network's first layer takes them (the same FP32 operations and rounding as its own
 // normalization; column 15 is 1).  Each wave owns a segment of kSegRows rows of Xb, one row
@@ -1017,7 +1017,7 @@ constexpr size_t kCountDoubles = sizeof(BatchCounts) / sizeof(double);
 static_assert(kCountDoubles * sizeof(double) == sizeof(BatchCounts), "whole doubles");
 static_assert(35 * sizeof(double) + sizeof(BatchCounts) + kListBytes + sizeof(uint32_t) <= 105 * sizeof(double),
               "a batch's scratch fits the fluxes");
-// A kernel rather than a memset, so that the launch sequence can be captured in a graph.
+// The counters start at zero, on the stream of the kernels that count.
 __global__ void k_batch_begin(BatchCounts* n) {
   clear_counts(&n->step);
   for (int r = 0; r <= kWideRounds; ++r) n->wide[r] = 0ull;

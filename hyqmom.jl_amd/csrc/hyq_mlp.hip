@@ -491,7 +491,7 @@ constexpr int NBIAS = 3 * HID + OUT + 1;  // bias gradients b1 b2 b3 b4 and the 
 constexpr int kRowWaves = 4;
 
 // One wave per 16 rows: forward (as the fused inference), loss gradient, and back to dZ1,
-// with the pre-activations in registers; writes the operands of the weight gradients and the
+// with the pre-activations in registers (at width 128 all 512 of a lane, and 328 B of scratch); writes the operands of the weight gradients and the
 // block's part of the bias gradients and the loss.  Rows past n (up to npad) give zeros.
 __global__ __launch_bounds__(64 * kRowWaves) void k_train_rows(
     const float* __restrict__ X, const float* __restrict__ T, long n, long npad,

@@ -13,8 +13,9 @@
 //   relax    projection and BGK of A
 // The one-kernel-per-pass form this replaces kept every path of a cell in one kernel: 0.6 to
 // 1.1 MB of code against an instruction cache of 64 KB shared by two CUs, with 1 KB of
-// scratch per lane.  These kernels are 8 to 108 KB each, with 240 B of scratch that only the
-// realizability edge branch touches.  Per step (pass 1 + pass 2, one kernel per pass -> this
+// scratch per lane.  These kernels are 8 to 109 KB each.  Those that project have 240 B of
+// scratch for the realizability edge branch; the two-wave forms for long lists spill beyond
+// that (k_hard 496 and 320 B, k_wide_close 272, k_wide_solve 448 with EM 1), the others do not.  Per step (pass 1 + pass 2, one kernel per pass -> this
 // form): 20x20x10 FP64 389 + 267 -> 150 + 143 us; 37x29x17 mixed 468 + 274 -> 260 + 185;
 // 120x120x60 FP64 1557 + 1082 -> 1336 + 964, learned 1830 -> 1306 in all.  What is left is the
 // latency of the serial root iterations (at 1 to 4 waves a SIMD) and, on small grids, of one

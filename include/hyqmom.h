@@ -227,7 +227,7 @@ int hyq_mlp_get_blob(hyq_mlp* m, float* blob_host);
 int hyq_mlp_set_blob(hyq_mlp* m, const float* blob_host);
 /* X [n][16] features (device), P [n][2] predictions (device): the fused inference kernel. */
 int hyq_mlp_infer(hyq_mlp* m, const float* X, int64_t n, float* P);
-/* the same through the layer-by-layer training kernels (bitwise equal; a cross-check) */
+/* the same through a kernel per layer (bitwise equal; a cross-check) */
 int hyq_mlp_infer_layers(hyq_mlp* m, const float* X, int64_t n, float* P);
 /* launch shape of the fused inference: -1 (the default) times the shapes on the first
  * inference of 65536 rows or more and keeps the fastest; 0..2 fixes one (0: 16 waves x 1
