@@ -1022,10 +1022,14 @@ __global__ void k_batch_begin(BatchCounts* n) {
   clear_counts(&n->step);
   for (int r = 0; r <= kWideRounds; ++r) n->wide[r] = 0ull;
 }
-// Batches from this size on take their entries through a launch per phase: with most cells on
-// the list (mixtures), one kernel that does every phase of a cell waits on its slowest lane
-// at 1 wave a SIMD.  524288 mixture cells in FP64: the whole batch 10.2 ms with k_hard, 6.75
-// ms wide (7.45 ms as one kernel per pass).
+// Batches from this size on take their entries through a launch per phase, 13 launches for one.
+// The number of entries, which decides what is faster, is known on the device only; with few
+// of them the launches cost 45 us.  us, k_hard / wide, by cells:
+//                  131072       160000       199999       262144       400000       1000000
+//   mixtures FP64  2008 / 2258  2643 / 2637  3649 / 3192  3677 / 3780  5920 / 5347  13713 / 11836
+//            fast  1676 / 1776  2362 / 2144  2545 / 2634  3100 / 2814  4688 / 4176  11107 / 9278
+//   jets     FP64   487 / 521    662 / 701    822 / 869    828 / 866   1215 / 1253   2568 / 2594
+//            fast   218 / 261    266 / 301    323 / 373    338 / 372    452 / 497     959 / 957
 constexpr long long kWideCells = 200000;
 static_assert(35 * sizeof(double) + sizeof(BatchCounts) / 1000 + kListBytes + sizeof(uint32_t) + kWideBytes <=
                   105 * sizeof(double), "a large batch's scratch fits the fluxes");
