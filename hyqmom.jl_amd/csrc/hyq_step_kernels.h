@@ -214,7 +214,8 @@ __device__ __forceinline__ void sort_out(const CellCtx& x, int lane, bool zs, co
 //     for another (with five waves to a block the other form keeps 1.1 waves per SIMD of the
 //     two that fit).
 // EM 1: P the network's seeds, or null.
-// Lanes.  8, 16 and 32 take the same time; 1: a 120x120x60 step on jets 3% more, 100000 jets
+//
+// kManyComplex: lanes.  8, 16 and 32 take the same time; 1: a 120x120x60 step on jets 3% more, 100000 jets
 // cells as a batch 482 -> 512 us; never: 100000 mixture cells 1831 -> 2092 us, 1000000 11.8
 // -> 13.1 ms.
 constexpr int kManyComplex = 16;
