@@ -848,13 +848,18 @@ __global__ __launch_bounds__(B, kProjWaves) void k_relax(Run R, double* __restri
 // Below so many blocks of 64 cells the planes of a cell are spread over waves.  The pass, in us,
 // spread / in turn, by blocks:
 //                  286          1025         1404         2052         4096        13500
-//   FP64   pass 1  229 / 369    400 / 433    490 / 483    613 / 551    988 / 738  1965 / 1336
-//          pass 2  180 / 304    245 / 320    279 / 351    338 / 396    535 / 554   979 / 964
+//   FP64   pass 2  180 / 304    245 / 320    279 / 351    338 / 396    535 / 554   979 / 964
 //   fast   pass 1  123 / 145    174 / 177    202 / 202    243 / 236    370 / 323
 //          pass 2  112 / 119    122 / 130    133 / 138    169 / 171    233 / 228
 // (Pass 1 spreads over five waves a block, of which fewer fit than of pass 2's four.)
+// FP64 pass 1, from as many blocks as there are SIMDs on in turn, on jets at Ma 0.7 and 1.5 and as
+// a batch of mixture cells:
+//          708          927          1000         1051         1131         1214         1422
+//   0.7    419 / 477    466 / 522    474 / 490    517 / 511    544 / 558    572 / 537    628 / 580
+//   1.5    412 / 469    478 / 519    472 / 479    513 / 499    550 / 537    579 / 540    638 / 581
+//   batch 1390 / 1240  1570 / 1345  1605 / 1370  1670 / 1405  1820 / 1715  2020 / 1728  2153 / 1736
 template <int EM, int PASS>
-constexpr unsigned kSpreadBelow = PASS == 1 ? 1280 : (EM == 0 ? 4096 : 2048);
+constexpr unsigned kSpreadBelow = PASS == 1 ? (EM == 0 ? 1024 : 1280) : (EM == 0 ? 4096 : 2048);
 // Launches of one pass after its projection (pass 1 up to k_hard, pass 2 up to k_hard).
 template <int EM, int PASS, typename FT, typename Run>
 void launch_planes(hipStream_t s, const Run& R, unsigned blocks64, double* A, FT* vp, uint32_t* flags,
