@@ -1,4 +1,7 @@
-// The per-cell passes of one time step (simulation_runner.jl:352-380 and :526-556).
+// The per-cell passes of one time step (simulation_runner.jl:352-380 and :526-556).  The kernels run
+// them in pieces (hyq_step_kernels.h); pass1_cell, pass2_cell and what only they call
+// (plane_solve, eig6_axis, eig6_z) are the whole of a cell in one function, for the host's parity
+// tests and the operation counter.  The kernels are held against the oracle on the device.
 #pragma once
 #include "hyq_fasteig.h"
 
