@@ -5,7 +5,7 @@
 // and eight threads copy between it and pageable memory faster than that, page faults
 // included.  So large copies go through a ring of pinned chunks, filled or emptied by threads
 // beside the transfers.  Pinned and device pointers, small arrays, and an object's first copies
-// below 64 MiB (early) are copied by the runtime as they are.  Down to fresh pages, in ms (runtime
+// below 24 MiB (early) are copied by the runtime as they are.  Down to fresh pages, in ms (runtime
 // / ring, once it is pinned): 9 MB 0.52 / 0.46, 16 MB 0.89 / 0.66, 34 MB 3.3 / 1.15, 68 MB 6.4 /
 // 1.9, 242 MB 22.6 / 5.6; up: 9 MB 0.26 / 0.36, 34 MB 1.04 / 0.97, 108 MB 3.7 / 2.6, 242 MB 8.3 / 5.4.
 #pragma once
@@ -48,25 +48,26 @@ class HostCopy {
     if (!staged(dst, bytes, kMin) || early(bytes))
       return direct(dst, src, bytes, hipMemcpyDeviceToHost, s);
     std::lock_guard<std::mutex> lk(mu_);
-    const size_t chunk = chunk_of(bytes);
-    Team t(static_cast<long>((bytes + chunk - 1) / chunk));
+    const Shape r = shape_of(bytes);
+    const size_t chunk = r.chunk;
+    Team t(static_cast<long>((bytes + chunk - 1) / chunk), r.slots);
     if (!pin() || !t.start([&](long k) {  // ready: its chunk has arrived
-          std::memcpy((char*)dst + k * chunk, slot(k, chunk), std::min(chunk, bytes - k * chunk));
+          std::memcpy((char*)dst + k * chunk, slot(k, r), std::min(chunk, bytes - k * chunk));
         }))
       return direct(dst, src, bytes, hipMemcpyDeviceToHost, s);
     long issued = 0;
     for (long k = 0; k < t.n; ++k) {
       // every transfer whose slot is empty, chunk k's in any case
-      for (; issued < t.n && issued < k + kSlots; ++issued) {
-        if (issued >= kSlots && !t.is_done(issued - kSlots)) {
+      for (; issued < t.n && issued < k + r.slots; ++issued) {
+        if (issued >= r.slots && !t.is_done(issued - r.slots)) {
           if (issued > k) break;
-          t.wait_done(issued - kSlots);
+          t.wait_done(issued - r.slots);
         }
-        const hipError_t e = move(slot(issued, chunk), (const char*)src + issued * chunk,
-                                  std::min(chunk, bytes - issued * chunk), hipMemcpyDeviceToHost, s, issued);
+        const hipError_t e = move(slot(issued, r), (const char*)src + issued * chunk,
+                                  std::min(chunk, bytes - issued * chunk), hipMemcpyDeviceToHost, s, issued % r.slots);
         if (e != hipSuccess) return stop(t, s, e);
       }
-      const hipError_t e = hipEventSynchronize(ev_[k % kSlots]);
+      const hipError_t e = hipEventSynchronize(ev_[k % r.slots]);
       if (e != hipSuccess) return stop(t, s, e);
       t.ready.store(k + 1, std::memory_order_release);
     }
@@ -76,22 +77,23 @@ class HostCopy {
   hipError_t to_device(void* dst, const void* src, size_t bytes, hipStream_t s) {
     if (!staged(src, bytes, kMinUp)) return direct(dst, src, bytes, hipMemcpyHostToDevice, s);
     std::lock_guard<std::mutex> lk(mu_);
-    const size_t chunk = chunk_of(bytes);
-    Team t(static_cast<long>((bytes + chunk - 1) / chunk));
+    const Shape r = shape_of(bytes);
+    const size_t chunk = r.chunk;
+    Team t(static_cast<long>((bytes + chunk - 1) / chunk), r.slots);
     if (!pin() || !t.start([&](long k) {  // ready: its slot is free
-          std::memcpy(slot(k, chunk), (const char*)src + k * chunk, std::min(chunk, bytes - k * chunk));
+          std::memcpy(slot(k, r), (const char*)src + k * chunk, std::min(chunk, bytes - k * chunk));
         }))
       return direct(dst, src, bytes, hipMemcpyHostToDevice, s);
-    t.ready.store(std::min<long>(kSlots, t.n), std::memory_order_release);
+    t.ready.store(std::min<long>(r.slots, t.n), std::memory_order_release);
     for (long k = 0; k < t.n; ++k) {
       t.wait_done(k);
-      hipError_t e = move((char*)dst + k * chunk, slot(k, chunk), std::min(chunk, bytes - k * chunk),
-                          hipMemcpyHostToDevice, s, k);
+      hipError_t e = move((char*)dst + k * chunk, slot(k, r), std::min(chunk, bytes - k * chunk),
+                          hipMemcpyHostToDevice, s, k % r.slots);
       // a slot is free again when its transfer is done: half a ring behind the newest
-      const long f = k - kSlots / 2;
-      if (e == hipSuccess && f >= 0 && f + kSlots < t.n) {
-        e = hipEventSynchronize(ev_[f % kSlots]);
-        t.ready.store(f + kSlots + 1, std::memory_order_release);
+      const long f = k - r.slots / 2;
+      if (e == hipSuccess && f >= 0 && f + r.slots < t.n) {
+        e = hipEventSynchronize(ev_[f % r.slots]);
+        t.ready.store(f + r.slots + 1, std::memory_order_release);
       }
       if (e != hipSuccess) return stop(t, s, e);
     }
@@ -100,12 +102,12 @@ class HostCopy {
   }
 
  private:
-  static constexpr long kSlots = 10;
+  static constexpr long kSlots = 10;  // at most
   static constexpr unsigned kThreads = 8;  // 4: a fresh 242 MB takes 5.2 ms, 8: 3.5, 12: 4.4
 
   // Threads that take chunks 0 .. n - 1 in turn, each as soon as `ready` passes it.
   struct Team {
-    explicit Team(long n_) : n(n_) {}
+    Team(long n_, long slots_) : n(n_), slots(slots_) {}
     ~Team() {
       quit.store(true);
       join();
@@ -124,14 +126,14 @@ class HostCopy {
                 std::this_thread::yield();
               }
               f(k);
-              last[k % kSlots].store(k + 1, std::memory_order_release);
+              last[k % slots].store(k + 1, std::memory_order_release);
             }
           });
       } catch (...) {  // fewer threads
       }
       return size > 0;
     }
-    bool is_done(long k) const { return last[k % kSlots].load(std::memory_order_acquire) > k; }
+    bool is_done(long k) const { return last[k % slots].load(std::memory_order_acquire) > k; }
     void wait_done(long k) const {
       while (!is_done(k)) std::this_thread::yield();
     }
@@ -139,7 +141,7 @@ class HostCopy {
       for (unsigned i = 0; i < size; ++i) team[i].join();
       size = 0;
     }
-    const long n;
+    const long n, slots;
     std::atomic<long> next{0}, ready{0};
     std::atomic<long> last[kSlots] = {};  // the latest chunk done in each slot, plus 1
     std::atomic<bool> quit{false};
@@ -157,15 +159,14 @@ class HostCopy {
     return true;
   }
   // Whether an object's copy down comes too early for the ring: pinning it and giving it back
-  // (in part paid by the next allocation) takes 0.3 to 3 ms, by what pages the system has at
-  // hand, and a copy saves 0.05 ms at 9 MB, 0.23 at 16 and 2.1 at 34.  So below 64 MiB the
-  // ring is for objects that have copied about as often as it takes to make up for that: 13
-  // times at 9 MB, 4 at 16, twice at 25, once from 30 MB on.  An object that copies once
-  // (create, a state up, one down, destroy), ring at once / runtime, ms: 9 MB 1.4 to 2.4 /
-  // 1.0, 16 MB 2.4 to 3.5 / 1.6, 34 MB 3.7 to 6.1 / 5.4, 56 MB 8.0 to 8.7 / 8.4, 68 MB 5.2 to
-  // 9.0 / 9.9.
+  // (in part paid by the next allocation) takes 0.3 to 1.3 ms at 12 MiB, by what pages the
+  // system has at hand, and a copy saves 0.05 ms at 9 MB, 0.23 at 16, 1.0 at 31 and 2.1 at 34.
+  // So below 24 MiB the ring is for objects that have copied about as often as it takes to
+  // make up for that: 13 times at 9 MB, 4 at 16, twice at 24.  An object that copies once
+  // (create, a state up, one down, destroy), ring at once / runtime, ms: 9 MB 1.4 to 2.4 / 1.0,
+  // 16 MB 2.4 to 3.5 / 1.6, 34 MB 3.7 to 5.6 / 5.4, 56 MB 5.4 / 8.5, 68 MB 5.0 to 9.6 / 9.7.
   bool early(size_t bytes) {
-    if (bytes >= kMinUp) return false;
+    if (bytes >= (size_t(24) << 20)) return false;
     const double r = double(size_t(32) << 20) / bytes;
     const int n = early_.load();
     if (n >= std::max(1, (int)(r * r + 0.5))) return false;
@@ -174,20 +175,27 @@ class HostCopy {
   }
   bool pin() {
     if (pin_) return true;
-    if (hipHostMalloc((void**)&pin_, chunk_of(max_) * kSlots, hipHostMallocPortable) == hipSuccess) return true;
+    if (hipHostMalloc((void**)&pin_, ring_of(max_), hipHostMallocPortable) == hipSuccess) return true;
     (void)hipGetLastError();
     pin_ = nullptr;
     return false;
   }
-  // 1 to 4 MiB, sixteen to a copy: a chunk costs the issuing thread 34 us, the transfer of 2 MB.
-  static size_t chunk_of(size_t bytes) {
-    const size_t c = (bytes / 16 + 4095) / 4096 * 4096;
-    return std::min(std::max(c, size_t(1) << 20), size_t(4) << 20);
+  struct Shape {
+    size_t chunk;
+    long slots;
+  };
+  // A chunk costs the issuing thread 34 us, the transfer of 2 MB.  Smaller copies take a smaller
+  // ring, whose pinning they make up for: 34 MB with 2 MiB x 6 1.17 ms a copy, x 4 1.37, x 8
+  // 1.12, 1 MiB x 8 1.32, 1.5 MiB x 6 1.22; 56 MB with 2 MiB x 6 2.2, x 8 1.9.
+  static Shape shape_of(size_t bytes) {
+    if (bytes >= kMinUp) return {size_t(4) << 20, kSlots};
+    return {size_t(2) << 20, bytes < (size_t(48) << 20) ? 6 : 8};
   }
-  char* slot(long k, size_t chunk) const { return pin_ + (size_t)(k % kSlots) * chunk; }
-  hipError_t move(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s, long k) {
+  static size_t ring_of(size_t bytes) { return shape_of(bytes).chunk * shape_of(bytes).slots; }
+  char* slot(long k, const Shape& r) const { return pin_ + (size_t)(k % r.slots) * r.chunk; }
+  hipError_t move(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s, long at) {
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, s);
-    return e != hipSuccess ? e : hipEventRecord(ev_[k % kSlots], s);
+    return e != hipSuccess ? e : hipEventRecord(ev_[at], s);
   }
   static hipError_t direct(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, s);
