@@ -186,9 +186,10 @@ class HostCopy {
   };
   // A chunk costs the issuing thread 34 us, the transfer of 2 MB.  Smaller copies take a smaller
   // ring, whose pinning they make up for: 34 MB with 2 MiB x 6 1.17 ms a copy, x 4 1.37, x 8
-  // 1.12, 1 MiB x 8 1.32, 1.5 MiB x 6 1.22; 56 MB with 2 MiB x 6 2.2, x 8 1.9.
+  // 1.12, 1 MiB x 8 1.32, 1.5 MiB x 6 1.22; 56 MB with 2 MiB x 6 2.2, x 8 1.9; 62 MB with 2 MiB
+  // x 8 0.4 ms more than with 4 MiB x 10.
   static Shape shape_of(size_t bytes) {
-    if (bytes >= kMinUp) return {size_t(4) << 20, kSlots};
+    if (bytes >= (size_t(56) << 20)) return {size_t(4) << 20, kSlots};
     return {size_t(2) << 20, bytes < (size_t(48) << 20) ? 6 : 8};
   }
   static size_t ring_of(size_t bytes) { return shape_of(bytes).chunk * shape_of(bytes).slots; }

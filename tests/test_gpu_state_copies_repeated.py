@@ -9,7 +9,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("N", [(32, 32, 30), (40, 40, 36), (45, 44, 43), (47, 46, 41), (61, 53, 37), (56, 56, 55), (60, 60, 57)])
+@pytest.mark.parametrize("N", [(32, 32, 30), (40, 40, 36), (45, 44, 43), (47, 46, 41), (61, 53, 37), (56, 56, 55), (60, 60, 57), (61, 60, 59)])
 def test_repeated_reads(N):
     import hyqmom_amd as H
     from hyqmom_amd.ensemble import jets_params
